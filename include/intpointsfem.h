@@ -158,8 +158,11 @@ int ipf_info(const ipf_ctx *ctx, int64_t out[8]);
  * (TPZElastoPlasticIntPointsStructMatrix.cpp:137-154) ->
  * TPZNumericalIntegrator::ResidualIntegration (TPZNumericalIntegrator.cpp:107-128).
  * One fused kernel per element color: gather, B.u, return map, B^T (w sigma)
- * and the color's atomic-free accumulation into r.  r is overwritten
- * entirely (its previous contents are never read); u and r must not
+ * and the color's atomic-free accumulation into r -- or, up to 2.5 million
+ * points of geometric B with aligned (x, y) DoF pairs in at most 8 colors, one
+ * element launch per shape and one node launch that sums in color order (the
+ * same bits; calls that overlap on several streams, and calls under capture,
+ * keep the launch per color).  r is overwritten entirely (its previous contents are never read); u and r must not
  * overlap.  Asynchronous on the context's stream. */
 int ipf_residual(ipf_ctx *ctx, const double *u_dev, double *r_dev);
 int ipf_residual_host(ipf_ctx *ctx, const double *u_host, double *r_host);
@@ -260,8 +263,8 @@ int ipf_certify_elastic_host(int64_t n, const double *strain3, const double *pla
                              double mu, double mc_phi, double mc_psi, double mc_cohesion, int *certified,
                              double *sigma3);
 
-/* ipf_residual with a HIP event pair around every kernel launch on the
- * context's stream; waits, then writes the duration of each launch in
+/* ipf_residual by its launch per color (or patch), with a HIP event pair
+ * around every kernel launch on the context's stream; waits, then writes the duration of each launch in
  * milliseconds to launch_ms (launch 0: r = f_lin copy, exactly 0 when no
  * copy runs, then one per element group in launch order) and the group's
  * point count to launch_pts (may be NULL).  With the patch assembly

@@ -17,6 +17,7 @@ SOURCES = [
     "ipf_kernels.hip",
     "ipf_solver.hip",
     "ipf_kernels_fmt.hip",
+    "ipf_split.hip",
     "ipf_assemble.hip",
     "ipf_pattern.hip",
     "ipf_learned.hip",

@@ -22,6 +22,7 @@
 #include "ipf_kernels.h"
 #include "ipf_learned.h"
 #include "ipf_patch.h"
+#include "ipf_split.h"
 
 namespace ipf {
 
@@ -238,6 +239,19 @@ struct ipf_ctx {
     // per element slot and node, the node's x DoF (y = x + 1), flagged like
     // dDofR, when every element's DoFs come in such pairs (GroupDev::node)
     int* dNodeR = nullptr;
+    // element / node launches (ipf_split.h): the launch of each shape, the
+    // nodes' element entries, the element forces.  dEf serves the calls of one
+    // stream at a time (split_stream); the CG's is its own (dEfS, with the
+    // solver buffers)
+    bool split_ok = false;
+    int map_stride = 0;
+    SplitDev split[SHAPE_COUNT];
+    int* dMap = nullptr;
+    double* dEf = nullptr;
+    double* dEfS = nullptr;
+    int64_t nent = 0;           // node entries of all element slots
+    bool ef_bound = false;
+    hipStream_t ef_stream = nullptr;
     double* dU = nullptr;       // staging for host-pointer calls
     double* dR = nullptr;
     int64_t bytes = 0;
@@ -266,7 +280,9 @@ struct ipf_ctx {
     double* dNt = nullptr;      // the Newton step while the Thomas correction is solved
     bool newton_thomas = false; // ipf_set_newton_thomas
     double* dPartial = nullptr; // dot partials
-    double* dScal = nullptr;    // CG scalars
+    double* dScal = nullptr;    // CG scalars (kRzEven ...)
+    double* hScal = nullptr;    // pinned: the scalars, then block partials that kernels write
+    double* dCp2 = nullptr;     // the CG's second direction buffer
     bool have_mask = false;
 
     // alternative B formats (index FMT_*; FMT_D64 is dB, FMT_G64 stores nothing)
@@ -370,6 +386,13 @@ void release_patch(ipf_ctx* ctx) {
     ctx->patch_built = false;
 }
 
+void release_split(ipf_ctx* ctx) {
+    dev_free(ctx->dMap);
+    dev_free(ctx->dEf);
+    ctx->split_ok = false;
+    ctx->ef_bound = false;
+}
+
 void release_data(ipf_ctx* ctx) {
     drop_cg_graph(ctx);
     release_patch(ctx);
@@ -389,6 +412,8 @@ void release_data(ipf_ctx* ctx) {
     dev_free(ctx->dDofR);
     ctx->fold_flin = false;
     dev_free(ctx->dNodeR);
+    release_split(ctx);
+    dev_free(ctx->dEfS);
     dev_free(ctx->dU);
     dev_free(ctx->dR);
     dev_free(ctx->dDep);
@@ -411,6 +436,7 @@ void release_data(ipf_ctx* ctx) {
     dev_free(ctx->dNt);
     dev_free(ctx->dPartial);
     dev_free(ctx->dScal);
+    dev_free(ctx->dCp2);
     for (int f = 1; f < FMT_COUNT; f++) dev_free(ctx->dBf[f]);
     dev_free(ctx->dGeo);
     dev_free(ctx->dTab);
@@ -435,6 +461,27 @@ void release_data(ipf_ctx* ctx) {
     ctx->bytes = 0;
 }
 
+// Up to how many points a residual or a CG iteration (and a single product)
+// takes the element / node launches.  Below, a color's launch leaves most of
+// the chip idle and the launches' own times add up; above, the element forces
+// no longer stay in the Infinity Cache and their write and read cost what the
+// colored launches' repeated r costs.  us per residual, colored -> element /
+// node: Q2 14 k points 23.2 -> 9.7, 90 k 25.3 -> 12.3, 810 k 58.6 -> 45.6,
+// 1.44 M 82.7 -> 73.8, 2.7 M 129.7 -> 127.9, 5.8 M 253 -> 264; Q1 2.56 M
+// 106 -> 100; Q3 2.56 M 159 -> 154.  Per CG iteration (nine launches -> three):
+// Q2 14 k 23.8 -> 12.9, 90 k 29.1 -> 16.8, 1.44 M 100.6 -> 85.1, 2.7 M 152 ->
+// 144, 5.8 M 280 -> 315.  Per product: 90 k 17.1 -> 9.0, 810 k 35.3 -> 32.1,
+// 2.7 M 87.9 -> 90.1; right after a residual and tangent (cold caches) 1.44 M
+// points already lose 2 us.
+constexpr int64_t kSplitPoints = 2500000, kSplitPointsProduct = 1000000;
+
+// Whether the CG takes the element / node launches (three per iteration).
+bool cg_split(const ipf_ctx* ctx) {
+    return ctx->split_ok && ctx->npad <= kSplitPoints && format_geometric(ctx->tfmt);
+}
+
+constexpr int kScal = 16;  // CG / Newton scalars in dScal
+
 // Solver workspace, allocated once per transferred data set.
 int ensure_solver_buffers(ipf_ctx* ctx) {
     if (ctx->dDep) return IPF_OK;
@@ -446,16 +493,26 @@ int ensure_solver_buffers(ipf_ctx* ctx) {
         (rc = dev_alloc(ctx, &ctx->dCr, ctx->neq)) || (rc = dev_alloc(ctx, &ctx->dCz, ctx->neq)) ||
         (rc = dev_alloc(ctx, &ctx->dCp, ctx->neq)) || (rc = dev_alloc(ctx, &ctx->dCq, ctx->neq)) ||
         (rc = dev_alloc(ctx, &ctx->dNr, ctx->neq)) || (rc = dev_alloc(ctx, &ctx->dNd, ctx->neq)) ||
-        (rc = dev_alloc(ctx, &ctx->dPartial, 1024)) || (rc = dev_alloc(ctx, &ctx->dScal, 16))) {
+        (rc = dev_alloc(ctx, &ctx->dPartial, 2048)) || (rc = dev_alloc(ctx, &ctx->dScal, kScal))) {
         return rc;
     }
     IPF_HIP(ctx, hipMemset(ctx->dDep, 0, sizeof(double) * 9 * ctx->npad));
-    IPF_HIP(ctx, hipMemset(ctx->dScal, 0, sizeof(double) * 16));
+    IPF_HIP(ctx, hipMemset(ctx->dScal, 0, sizeof(double) * kScal));
     if (!ctx->dMask) {
         if ((rc = dev_alloc(ctx, &ctx->dMask, ctx->neq))) return rc;
         IPF_HIP(ctx, hipMemset(ctx->dMask, 0, ctx->neq));
     }
     return IPF_OK;
+}
+
+// What only a CG needs beside them: the pinned scalars and, for the element /
+// node launches, its element forces and second direction buffer.
+int ensure_cg_buffers(ipf_ctx* ctx) {
+    if (!ctx->hScal) IPF_HIP(ctx, hipHostMalloc((void**)&ctx->hScal, sizeof(double) * (kScal + 1024), 0));
+    if (!cg_split(ctx) || ctx->dCp2) return IPF_OK;
+    int rc;
+    if (!ctx->dEfS && (rc = dev_alloc(ctx, &ctx->dEfS, 2 * ctx->nent))) return rc;
+    return dev_alloc(ctx, &ctx->dCp2, ctx->neq);
 }
 
 int read_scalar(ipf_ctx* ctx, int slot, double* out) {
@@ -665,6 +722,85 @@ const double* residual_start(ipf_ctx* ctx, double* r) {
     return nullptr;
 }
 
+// The launches and the node map of the element / node launches: geometric
+// data whose elements number their nodes' DoFs as aligned (x, y) pairs, in at
+// most 8 colors.  Out of memory leaves the colored launches (not an error).
+void build_split(ipf_ctx* ctx) {
+    const int stride = ctx->ncolor <= 4 ? 4 : 8;
+    int64_t nent = 0, ntile = 0;
+    for (const auto& g : ctx->groups) {
+        nent = std::max(nent, g.dof_off / 2 + (int64_t)g.elems.size() * (shape_ce(g.shape) / 2));
+        ntile += g.ntiles;
+    }
+    if (!ctx->have_geometry || !ctx->pairs_aligned || ctx->ncolor > kSplitColors || ntile == 0 || nent > INT32_MAX ||
+        ctx->npad > INT32_MAX)
+        return;
+    for (int sh = 0; sh < SHAPE_COUNT; sh++) {
+        SplitDev& d = ctx->split[sh];
+        d = SplitDev{};
+        if (ctx->tab_off[sh] < 0) continue;
+        const int ET = shape_et(sh), NE = ET * (shape_ce(sh) / 2), TP = shape_tp(sh);
+        for (const auto& g : ctx->groups) {
+            if (g.shape != sh) continue;
+            const int64_t t0 = d.ntiles;  // launch tile of the group's first
+            d.tile0[d.nseg] = (int)(g.tile0 - t0);
+            d.pt0[d.nseg] = (int)(g.pt0 - t0 * TP);
+            d.slot0[d.nseg] = (int)(g.slot0 - t0 * ET);
+            d.ent0[d.nseg] = (int)(g.dof_off / 2 - t0 * NE);
+            d.ntiles += g.ntiles;
+            d.end[d.nseg++] = (int)d.ntiles;
+        }
+        d.tmeta = ctx->dTmeta;
+        d.geo = ctx->dGeo;
+        d.tab = ctx->dTab + ctx->tab_off[sh];
+        d.node = ctx->dNodeR;
+    }
+    const int64_t nnode = (ctx->neq + 1) / 2;
+    const std::string err = ctx->err;
+    if (dev_alloc(ctx, &ctx->dMap, nnode * stride) || dev_alloc(ctx, &ctx->dEf, 2 * nent)) {
+        (void)hipGetLastError();
+        ctx->err = err;
+        release_split(ctx);
+        return;
+    }
+    launch_fill_int(nnode * stride, ctx->dMap, -1, ctx->stream);
+    for (const auto& g : ctx->groups) {
+        GroupDev d = group_dev(ctx, g);
+        d.node = ctx->dNodeR + g.dof_off / 2;
+        launch_node_map(g.shape, d, g.dof_off / 2, g.color, stride, ctx->dMap, ctx->stream);
+    }
+    ctx->map_stride = stride;
+    ctx->nent = nent;
+    ctx->split_ok = true;
+}
+
+// Whether a call on the context's stream may use dEf: calls of one stream are
+// ordered; another stream's calls could overlap with them (they keep the
+// colored launches until the first stream has been waited for), and so could
+// the replays of a graph that the caller captures.
+bool split_stream(ipf_ctx* ctx) {
+    if (!ctx->split_ok || ctx->stream == hipStreamPerThread) return false;
+    if (ctx->ef_bound && ctx->ef_stream != ctx->stream) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+    ctx->ef_bound = true;
+    ctx->ef_stream = ctx->stream;
+    return true;
+}
+
+SplitDev split_dev(const ipf_ctx* ctx, int sh) {
+    SplitDev d = ctx->split[sh];
+    d.mats = ctx->dMats;  // replaced by ipf_set_material_table
+    return d;
+}
+
+// the element forces of K v into ef
+void elem_tangent(ipf_ctx* ctx, const double* v, const CgBeta& cg, double* ef, hipStream_t s) {
+    for (int sh = 0; sh < SHAPE_COUNT; sh++)
+        if (ctx->split[sh].ntiles)
+            launch_elem_tangent(ctx->tfmt, sh, split_dev(ctx, sh), v, cg, ctx->dDep, ctx->dDep32, ctx->npad, ef, s);
+}
+
 // y = K v on stream s: the tangent launches of every group in the selected
 // B format.  When every DoF has a first write (fold_flin), the flagged entries
 // start from 0 and y needs no clear; else y is cleared first.
@@ -693,21 +829,57 @@ int ensure_dep32(ipf_ctx* ctx) {
     return IPF_OK;
 }
 
-constexpr int kCgBlock = 10;  // CG iterations between convergence checks
+constexpr int kCgBlock = 10;  // CG iterations between convergence checks (even: see kRzEven)
+// dScal: dots in slots 0..10; r.z of the iteration before at an even / odd
+// iteration of a block.  hScal: the scalars, then the block partials of r.r
+constexpr int kRzEven = 11, kRzOdd = 12;
 
-// `count` preconditioned CG iterations on stream s: q = K p (masked) and
-// p.q, alpha, x / r / z update and r.z, beta, new p.  The scalars stay on
-// the device, so the sequence has no host dependency.
+// Block partials of the CG's dots.  The element launch sums them in every
+// wavefront: at most 256 there.
+int cg_dot_blocks(const ipf_ctx* ctx) {
+    return cg_split(ctx) ? std::min(256, dot_blocks((ctx->neq + 1) / 2)) : dot_blocks(ctx->neq);
+}
+
+// `count` preconditioned CG iterations on stream s: p = z + beta p, q = K p
+// (masked) and p.q, x / r / z update and r.z, after the last one also r.r.
+// The scalars stay on the device, so the sequence has no host dependency.
+// With the element / node launches p alternates between two buffers: the node
+// launch writes the p that the element launch gathered from the other.
 void cg_iterations(ipf_ctx* ctx, double* x, int count, hipStream_t s) {
     const int64_t n = ctx->neq;
-    const int nb = dot_blocks(n);
+    const bool split = cg_split(ctx);
+    const int nb = cg_dot_blocks(ctx);
     for (int k = 0; k < count; k++) {
-        tangent_product(ctx, ctx->dCp, ctx->dCq, s);
-        launch_cg_mask_dot(n, ctx->dMask, ctx->dCp, ctx->dCq, ctx->dPartial, nb, ctx->dScal, s);
-        launch_cg_update_dot(n, ctx->dScal, ctx->dCp, ctx->dCq, x, ctx->dCr, ctx->dPa, ctx->dPb, ctx->dCz, ctx->dPartial,
-                             nb, s);
-        launch_cg_direction(n, ctx->dScal, ctx->dCz, ctx->dCp, s);
+        const double* rz_old = ctx->dScal + (k & 1 ? kRzOdd : kRzEven);
+        double* rz_new = ctx->dScal + (k & 1 ? kRzEven : kRzOdd);
+        double *pq = ctx->dPartial, *rz = ctx->dPartial + 1024;
+        double* p = split && (k & 1) == 0 ? ctx->dCp2 : ctx->dCp;
+        if (split) {
+            const CgBeta cg{(k & 1) == 0 ? ctx->dCp : ctx->dCp2, rz_old, rz, nb};
+            elem_tangent(ctx, ctx->dCz, cg, ctx->dEfS, s);
+            launch_nodes_cg(n, ctx->map_stride, ctx->dMap, ctx->dEfS, ctx->dMask, ctx->dCz, cg, rz_new, p, ctx->dCq, pq,
+                            nb, s);
+        } else {
+            launch_cg_direction(n, rz_old, rz_new, rz, nb, ctx->dCz, p, s);
+            tangent_product(ctx, p, ctx->dCq, s);
+            launch_cg_mask_dot(n, ctx->dMask, p, ctx->dCq, pq, nb, s);
+        }
+        launch_cg_update_dot(n, rz_new, pq, nb, p, ctx->dCq, x, ctx->dCr, ctx->dPa, ctx->dPb, ctx->dCz, rz,
+                             k == count - 1 ? ctx->hScal + kScal : nullptr, nb, s);
     }
+}
+
+// ||r||^2 after a block of CG iterations -- the block's last kernel leaves its
+// partials in pinned memory, summed here -- and (v set) the scalars [0, kScal).
+int read_rr(ipf_ctx* ctx, double* v, double* rr) {
+    if (v)
+        IPF_HIP(ctx, hipMemcpyAsync(ctx->hScal, ctx->dScal, sizeof(double) * kScal, hipMemcpyDeviceToHost, ctx->stream));
+    IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (v) std::copy(ctx->hScal, ctx->hScal + kScal, v);
+    double s = 0.0;
+    for (int i = 0; i < cg_dot_blocks(ctx); i++) s += ctx->hScal[kScal + i];
+    *rr = s;
+    return IPF_OK;
 }
 
 // The graph of kCgBlock iterations for iterate x (captured on the context's
@@ -866,6 +1038,7 @@ int ipf_ctx_destroy(ipf_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     release_data(ctx);
     dev_free(ctx->dMats);
+    if (ctx->hScal) (void)hipHostFree(ctx->hScal);
     if (ctx->cap_stream) (void)hipStreamDestroy(ctx->cap_stream);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
@@ -885,6 +1058,7 @@ int ipf_synchronize(ipf_ctx* ctx) {
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     IPF_HIP(ctx, hipGetLastError());
+    if (ctx->ef_stream == ctx->stream) ctx->ef_bound = false;  // nothing uses dEf any more
     return IPF_OK;
 }
 
@@ -1300,8 +1474,13 @@ static int transfer_impl(ipf_ctx* ctx, int64_t nblocks, const int* row_sizes, co
             release_data(ctx);
             return rc;
         }
-        IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
         ctx->have_geometry = true;
+        build_split(ctx);
+        if ((rc = launch_status(ctx, "node map"))) {
+            release_data(ctx);
+            return rc;
+        }
+        IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
     ctx->have_data = true;
     ctx->patch_in = std::move(pin);
@@ -1701,6 +1880,15 @@ int ipf_residual(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     if (!u_dev || !r_dev) return fail(ctx, IPF_EINVAL, "ipf_residual: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if (ctx->assembly == IPF_ASSEMBLY_PATCH && !ctx->update_mem) return patch_residual(ctx, u_dev, r_dev);
+    if (!ctx->update_mem && format_geometric(ctx->rfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
+        const PointState st = point_state(ctx);
+        for (int sh = 0; sh < SHAPE_COUNT; sh++)
+            if (ctx->split[sh].ntiles)
+                launch_elem_residual(ctx->rfmt, sh, ctx->residual_mode == IPF_RESIDUAL_CERTIFIED_ELASTIC,
+                                     split_dev(ctx, sh), u_dev, st, ctx->dEf, ctx->stream);
+        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, ctx->dFlin, r_dev, ctx->stream);
+        return launch_status(ctx, "residual");
+    }
     // r = f_lin, then each color adds -B^T(w sigma)
     const double* flin = residual_start(ctx, r_dev);
     const PointState st = point_state(ctx);
@@ -2049,8 +2237,8 @@ void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStre
 
 // The start of a CG solve of K x = b on stream s: the block-Jacobi
 // preconditioner of the current tangent (each node's 2x2 diagonal block
-// inverted where the DoFs pair up, else its diagonal), x = 0, r / z / p, r.z
-// into scalar 0 and ||r||^2 into scalar bb_slot.
+// inverted where the DoFs pair up, else its diagonal), x = 0, r / z / p, the
+// partials of r.z and ||r||^2 into scalar bb_slot.
 void cg_start(ipf_ctx* ctx, const double* b, double* x, int bb_slot, hipStream_t s) {
     const int64_t n = ctx->neq;
     const int nb = dot_blocks(n);
@@ -2062,8 +2250,9 @@ void cg_start(ipf_ctx* ctx, const double* b, double* x, int bb_slot, hipStream_t
     launch_block_jacobi(n, ctx->dMask, ctx->dDiag, offd, ctx->dPa, ctx->dPb, s);
     launch_fill(n, x, 0.0, s);
     launch_cg_init(n, ctx->dMask, b, ctx->dCr, ctx->dPa, ctx->dPb, ctx->dCz, ctx->dCp, s);
-    launch_dot(n, ctx->dCr, ctx->dCz, ctx->dPartial, nb, ctx->dScal + 0, s);
     launch_dot(n, ctx->dCr, ctx->dCr, ctx->dPartial, nb, ctx->dScal + bb_slot, s);
+    launch_dot_partials(n, ctx->dCr, ctx->dCz, ctx->dPartial + 1024, cg_dot_blocks(ctx), s);
+    launch_fill(1, ctx->dScal + kRzEven, 0.0, s);
 }
 
 // CG blocks from iteration *it (relative residual *rel there) on the
@@ -2071,8 +2260,6 @@ void cg_start(ipf_ctx* ctx, const double* b, double* x, int bb_slot, hipStream_t
 // block up to maxit launched one by one), ||r|| read after each block, until
 // it drops to rtol * bnorm (or turns NaN) or maxit is reached.
 int cg_blocks(ipf_ctx* ctx, double* x, double rtol, int maxit, double bnorm, int* it, double* rel) {
-    const int64_t n = ctx->neq;
-    const int nb = dot_blocks(n);
     hipStream_t s = ctx->stream;
     int rc;
     while (*it < maxit) {
@@ -2083,9 +2270,8 @@ int cg_blocks(ipf_ctx* ctx, double* x, double rtol, int maxit, double bnorm, int
         else
             cg_iterations(ctx, x, blk, s);
         *it += blk;
-        launch_dot(n, ctx->dCr, ctx->dCr, ctx->dPartial, nb, ctx->dScal + 3, s);
         double rr;
-        if ((rc = launch_status(ctx, "cg")) || (rc = read_scalar(ctx, 3, &rr))) return rc;
+        if ((rc = launch_status(ctx, "cg")) || (rc = read_rr(ctx, nullptr, &rr))) return rc;
         *rel = std::sqrt(rr) / bnorm;
         if (!(*rel > rtol)) break;  // also stops on NaN
     }
@@ -2097,7 +2283,7 @@ int cg_blocks(ipf_ctx* ctx, double* x, double rtol, int maxit, double bnorm, int
 // ipf_residual_tangent into r = dNr (and the FP32 copy of w Dep for the
 // FP32 geometric tangent), ||r||^2 over the free DoFs (scalar 6), the CG
 // start for K dNd = dNr with ||r||^2 in scalar 7, its first kCgBlock
-// iterations and ||r_cg||^2 (scalar 3).  The same kernels in the same order
+// iterations and ||r_cg||^2 (block partials).  The same kernels in the same order
 // as the eager iteration, so the iterates are the same bits.  nullptr when
 // capture fails (the caller then runs the iteration eagerly).  Needs the
 // solver buffers (and dDep32 for FMT_G32) allocated.
@@ -2116,7 +2302,6 @@ hipGraphExec_t newton_step_graph(ipf_ctx* ctx, const double* u) {
     masked_norm_launch(ctx, ctx->dNr, s);
     cg_start(ctx, ctx->dNr, ctx->dNd, 7, s);
     cg_iterations(ctx, ctx->dNd, kCgBlock, s);
-    launch_dot(ctx->neq, ctx->dCr, ctx->dCr, ctx->dPartial, dot_blocks(ctx->neq), ctx->dScal + 3, s);
     hipGraph_t graph = nullptr;
     const hipError_t e1 = hipStreamEndCapture(s, &graph);
     hipGraphExec_t exec = nullptr;
@@ -2307,7 +2492,12 @@ int ipf_tangent_apply(ipf_ctx* ctx, const double* v_dev, double* y_dev) {
     if (!v_dev || !y_dev) return fail(ctx, IPF_EINVAL, "ipf_tangent_apply: NULL pointer");
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    tangent_product(ctx, v_dev, y_dev, ctx->stream);
+    if (format_geometric(ctx->tfmt) && ctx->npad <= kSplitPointsProduct && split_stream(ctx)) {
+        elem_tangent(ctx, v_dev, CgBeta{}, ctx->dEf, ctx->stream);
+        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, nullptr, y_dev, ctx->stream);
+    } else {
+        tangent_product(ctx, v_dev, y_dev, ctx->stream);
+    }
     return launch_status(ctx, "tangent_apply");
 }
 
@@ -2319,7 +2509,7 @@ int ipf_cg_solve(ipf_ctx* ctx, const double* b_dev, double* x_dev, double rtol, 
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     if (!(rtol > 0) || maxit < 1) return fail(ctx, IPF_EINVAL, "ipf_cg_solve: need rtol > 0 and maxit >= 1");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if ((rc = ensure_solver_buffers(ctx))) return rc;
+    if ((rc = ensure_solver_buffers(ctx)) || (rc = ensure_cg_buffers(ctx))) return rc;
     if ((rc = ensure_dep32(ctx))) return rc;
     cg_start(ctx, b_dev, x_dev, 3, ctx->stream);
     double bb;
@@ -2341,7 +2531,7 @@ int ipf_newton(ipf_ctx* ctx, double* u_dev, double rtol, int maxit, double cg_rt
     if (ctx->newton_thomas && ctx->ls_halvings > 0)
         return fail(ctx, IPF_EINVAL, "ipf_newton: the Thomas acceleration and the line search exclude each other");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if ((rc = ensure_solver_buffers(ctx))) return rc;
+    if ((rc = ensure_solver_buffers(ctx)) || (rc = ensure_cg_buffers(ctx))) return rc;
     if (ctx->newton_thomas && !ctx->dNt && (rc = dev_alloc(ctx, &ctx->dNt, ctx->neq))) return rc;
     // The caller's UpdateMem switch is restored on every exit: the Newton
     // residuals must not commit, only the final AcceptPseudoTimeStepSolution.
@@ -2369,11 +2559,10 @@ int ipf_newton(ipf_ctx* ctx, double* u_dev, double rtol, int maxit, double cg_rt
             }
             ctx->have_tangent = true;
             ctx->dep32_ok = ctx->tfmt == FMT_G32;
-            double v[8];
-            if ((rc = launch_status(ctx, "newton step")) || (rc = read_scalars(ctx, 8, v))) break;
+            double v[kScal];
+            if ((rc = launch_status(ctx, "newton step")) || (rc = read_rr(ctx, v, &rr))) break;
             rn = std::sqrt(v[6]);
             bb = v[7];
-            rr = v[3];
         } else {
             if ((rc = ipf_residual_tangent(ctx, u_dev, ctx->dNr))) break;
             if ((rc = masked_norm(ctx, ctx->dNr, &rn))) break;

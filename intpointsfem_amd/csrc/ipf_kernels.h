@@ -52,6 +52,28 @@ __device__ __forceinline__ const MatConst& tile_material(const GroupDev& g, int6
     return g.mats[g.tmeta[tile] >> 8];
 }
 
+// The sum of n >= 1 partials in every lane of a wavefront, in one order; every
+// lane takes part.  The loads of the first 256 leave when the object is made,
+// so that they travel with the caller's other requests.
+struct WaveSum {
+    double v[4];
+    __device__ __forceinline__ WaveSum(int n, const double* __restrict__ partial) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = partial[min((int)(threadIdx.x & 63) + 64 * k, n - 1)];
+    }
+    __device__ __forceinline__ double get(int n, const double* __restrict__ partial) const {
+        const int lane = threadIdx.x & 63;
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s = lane + 64 * k < n ? s + v[k] : s;
+        for (int i = lane + 256; i < n; i += 64) s = s + partial[i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s = s + __shfl_xor(s, o, 64);
+        return s;
+    }
+};
+__device__ __forceinline__ double cg_beta(double rz, double rz_old) { return rz_old != 0.0 ? rz / rz_old : 0.0; }
+
 struct PointState {
     const double* w;
     double* ep0;          // plastic strain XX
@@ -197,17 +219,24 @@ void launch_cg_init(int64_t n, const signed char* mask, const double* b, double*
 // inverse of each node's 2x2 diagonal block, or Jacobi where none applies.
 void launch_block_jacobi(int64_t n, const signed char* mask, const double* diag, const double* offd, double* pa,
                          double* pb, hipStream_t stream);
-void launch_cg_mask(int64_t n, const signed char* mask, double* q, hipStream_t stream);
-void launch_cg_update(int64_t n, const double* scal, const double* p, const double* q, double* x, double* r,
-                      const double* pa, const double* pb, double* z, hipStream_t stream);
-void launch_cg_direction(int64_t n, const double* scal, const double* z, double* p, hipStream_t stream);
-// fused forms on the CG scalars scal (rz, pq, rz_new, ., alpha, beta):
-// q masked, pq = p.q and alpha = rz / pq; update with alpha, rz_new = r.z,
-// beta = rz_new / rz and rz = rz_new
+// One CG iteration: the kernels that need alpha or beta sum the block partials
+// of the dot behind it themselves (WaveSum), so the scalars need no launch of
+// their own.  r.z of the iteration before is *rz_old (0 before the first).
+//   direction: rz = sum of rz_partial, beta = rz / *rz_old, p = z + beta p,
+//              *rz_new = rz
+//   mask_dot:  q = 0 where mask is set, partials of p.q
+//   update:    alpha = *rz_new / p.q, x += alpha p, r -= alpha q, z = M r,
+//              partials of r.z and (rr_partial set) of r.r
+void launch_cg_direction(int64_t n, const double* rz_old, double* rz_new, const double* rz_partial, int nrz,
+                         const double* z, double* p, hipStream_t stream);
 void launch_cg_mask_dot(int64_t n, const signed char* mask, const double* p, double* q, double* partial, int nb,
-                        double* scal, hipStream_t stream);
-void launch_cg_update_dot(int64_t n, double* scal, const double* p, const double* q, double* x, double* r,
-                          const double* pa, const double* pb, double* z, double* partial, int nb, hipStream_t stream);
+                        hipStream_t stream);
+void launch_cg_update_dot(int64_t n, const double* rz_new, const double* pq_partial, int npq, const double* p,
+                          const double* q, double* x, double* r, const double* pa, const double* pb, double* z,
+                          double* rz_partial, double* rr_partial, int nb, hipStream_t stream);
+// block partials of x.y, as launch_dot's first kernel
+void launch_dot_partials(int64_t n, const double* x, const double* y, double* partial, int nblocks,
+                         hipStream_t stream);
 void launch_axpy(int64_t n, double a, const double* x, double* y, hipStream_t stream);
 // x = a x
 void launch_scale(int64_t n, double a, double* x, hipStream_t stream);

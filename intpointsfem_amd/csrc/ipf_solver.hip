@@ -3,9 +3,12 @@
 // main.cpp:283-285; its unused TPZCudaCalls::SolveCG, TPZCudaCalls.cu:213-290,
 // is a plain CG).  Dot products are FP64 with a fixed reduction order (block
 // partials in order, then one block), so repeated solves are bit-identical.
-// CG scalars live in a small device array so an iteration needs no host sync:
-//   scal[0] rz = r.z    scal[1] pq = p.q    scal[2] rz_new
-//   scal[3] rr = r.r    scal[4] alpha      scal[5] beta
+// The CG scalars alpha and beta live nowhere: the kernel that applies one sums
+// the block partials of its dot itself, in every block and in one order (at
+// most 1,024 values out of L2), so an iteration needs no host sync and no
+// launch for a scalar.  r.z of the iteration before is in device memory.
+#include <algorithm>
+
 #include "ipf_kernels.h"
 
 namespace ipf {
@@ -98,32 +101,6 @@ __global__ void k_block_jacobi(int64_t n, const signed char* __restrict__ mask, 
     }
 }
 
-__global__ void k_cg_mask(int64_t n, const signed char* __restrict__ mask, double* __restrict__ q) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && mask[i]) q[i] = 0.0;
-}
-
-__global__ void k_cg_update(int64_t n, const double* __restrict__ scal, const double* __restrict__ p,
-                            const double* __restrict__ q, double* __restrict__ x, double* __restrict__ r,
-                            const double* __restrict__ pa, const double* __restrict__ pb, double* __restrict__ z) {
-    const int64_t i0 = 2 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i0 >= n) return;
-    const int64_t i1 = i0 + 1;
-    const bool has1 = i1 < n;
-    const double alpha = scal[4];
-    x[i0] = x[i0] + alpha * p[i0];
-    const double r0 = r[i0] - alpha * q[i0];
-    r[i0] = r0;
-    double r1 = 0.0;
-    if (has1) {
-        x[i1] = x[i1] + alpha * p[i1];
-        r1 = r[i1] - alpha * q[i1];
-        r[i1] = r1;
-        z[i1] = pa[i1] * r1 + pb[i1] * r0;
-    }
-    z[i0] = pa[i0] * r0 + pb[i0] * r1;
-}
-
 // q = 0 on fixed DoFs, and the block partials of p.q (k_dot_partial's order)
 __global__ void __launch_bounds__(kDotThreads)
 k_cg_mask_dot(int64_t n, const signed char* __restrict__ mask, const double* __restrict__ p, double* __restrict__ q,
@@ -166,20 +143,61 @@ k_cg_mask_dot(int64_t n, const signed char* __restrict__ mask, const double* __r
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// k_cg_update and the block partials of r.z
+// x += alpha p, r -= alpha q, z = M r, the block partials of r.z and (RR) of r.r
+template <bool RR>
 __global__ void __launch_bounds__(kDotThreads)
-k_cg_update_dot(int64_t n, const double* __restrict__ scal, const double* __restrict__ p,
-                const double* __restrict__ q, double* __restrict__ x, double* __restrict__ r,
-                const double* __restrict__ pa, const double* __restrict__ pb, double* __restrict__ z,
-                double* __restrict__ partial) {
+k_cg_update_dot(int64_t n, const double* __restrict__ rz_new, const double* __restrict__ pq_partial, int npq,
+                const double* __restrict__ p, const double* __restrict__ q, double* __restrict__ x,
+                double* __restrict__ r, const double* __restrict__ pa, const double* __restrict__ pb,
+                double* __restrict__ z, double* __restrict__ partial, double* __restrict__ rr_partial) {
     __shared__ double sh[kDotThreads];
-    const double alpha = scal[4];
-    double s = 0.0;
+    double s = 0.0, rr = 0.0;
     // one DoF pair per thread and step (see k_cg_init); batches of U whole
     // pairs with every load in flight at once, then the same arithmetic and
     // the same order of the r.z terms as the loop below
     const int64_t S = (int64_t)gridDim.x * kDotThreads;
     int64_t k = (int64_t)blockIdx.x * kDotThreads + threadIdx.x;
+    // The thread's first pair is requested together with the partials of p.q
+    // and *rz_new: on a small mesh it is the only one, and its round trip
+    // hides behind theirs.
+    const WaveSum ws(npq, pq_partial);
+    const double rzv = *rz_new;
+    double v1[12];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int64_t i = min(2 * k + j, n - 1);
+        v1[6 * j] = x[i];
+        v1[6 * j + 1] = p[i];
+        v1[6 * j + 2] = q[i];
+        v1[6 * j + 3] = r[i];
+        v1[6 * j + 4] = pa[i];
+        v1[6 * j + 5] = pb[i];
+    }
+    const double pq = ws.get(npq, pq_partial);
+    const double alpha = pq != 0.0 ? rzv / pq : 0.0;
+    if (2 * k < n) {
+        const int64_t i0 = 2 * k, i1 = i0 + 1;
+        const bool has1 = i1 < n;
+        x[i0] = v1[0] + alpha * v1[1];
+        const double r0 = v1[3] - alpha * v1[2];
+        r[i0] = r0;
+        double r1 = 0.0;
+        if (has1) {
+            x[i1] = v1[6] + alpha * v1[7];
+            r1 = v1[9] - alpha * v1[8];
+            r[i1] = r1;
+        }
+        const double z0 = v1[4] * r0 + v1[5] * r1;
+        z[i0] = z0;
+        s = s + r0 * z0;
+        if (has1) {
+            const double z1 = v1[10] * r1 + v1[11] * r0;
+            z[i1] = z1;
+            s = s + r1 * z1;
+        }
+        if (RR) rr = (rr + r0 * r0) + r1 * r1;
+    }
+    k += S;
     constexpr int U = 2;
     for (; 2 * (k + (U - 1) * S) + 1 < n; k += U * S) {
         double xv[2 * U], pv[2 * U], qv[2 * U], rv[2 * U], av[2 * U], bv[2 * U];
@@ -210,6 +228,7 @@ k_cg_update_dot(int64_t n, const double* __restrict__ scal, const double* __rest
             const double z1 = av[j1] * r1 + bv[j1] * r0;
             z[i1] = z1;
             s = s + r1 * z1;
+            if (RR) rr = (rr + r0 * r0) + r1 * r1;
         }
     }
     for (; 2 * k < n; k += S) {
@@ -232,38 +251,27 @@ k_cg_update_dot(int64_t n, const double* __restrict__ scal, const double* __rest
             z[i1] = z1;
             s = s + r1 * z1;
         }
+        if (RR) rr = (rr + r0 * r0) + r1 * r1;
     }
     const double t = block_sum(s, sh);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
-}
-
-// p = z + beta p
-__global__ void k_cg_direction(int64_t n, const double* __restrict__ scal, const double* __restrict__ z,
-                               double* __restrict__ p) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    p[i] = z[i] + scal[5] * p[i];
-}
-
-// The block partials summed as k_dot_final does, then the CG scalars
-// (scal: rz, pq, rz_new, ., alpha, beta).  stage 0: pq = the sum, alpha =
-// rz / pq;  stage 1: rz_new = the sum, beta = rz_new / rz, rz = rz_new.
-__global__ void __launch_bounds__(kDotThreads)
-k_cg_final(int nb, const double* __restrict__ partial, double* __restrict__ scal, int stage) {
-    __shared__ double sh[kDotThreads];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nb; i += kDotThreads) s = s + partial[i];
-    const double t = block_sum(s, sh);
-    if (threadIdx.x != 0) return;
-    if (stage == 0) {
-        scal[1] = t;
-        scal[4] = t != 0.0 ? scal[0] / t : 0.0;
-    } else {
-        const double rz = scal[0];
-        scal[2] = t;
-        scal[5] = rz != 0.0 ? t / rz : 0.0;
-        scal[0] = t;
+    if (RR) {
+        __syncthreads();
+        const double t2 = block_sum(rr, sh);
+        if (threadIdx.x == 0) rr_partial[blockIdx.x] = t2;
     }
+}
+
+// rz = the sum of rz_partial, beta = rz / rz_old, p = z + beta p; rz is kept in
+// the other of two slots (the blocks read rz_old at their own pace)
+__global__ void __launch_bounds__(kDotThreads)
+k_cg_direction(int64_t n, const double* __restrict__ rz_old, double* __restrict__ rz_new,
+               const double* __restrict__ rz_partial, int nrz, const double* __restrict__ z, double* __restrict__ p) {
+    const double rz = WaveSum(nrz, rz_partial).get(nrz, rz_partial);
+    const double beta = cg_beta(rz, *rz_old);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *rz_new = rz;
+    const int64_t S = (int64_t)gridDim.x * kDotThreads;
+    for (int64_t i = (int64_t)blockIdx.x * kDotThreads + threadIdx.x; i < n; i += S) p[i] = z[i] + beta * p[i];
 }
 
 __global__ void k_axpy(int64_t n, double a, const double* __restrict__ x, double* __restrict__ y) {
@@ -322,15 +330,23 @@ void launch_segment_sumsq(const double* x, const signed char* mask, const int64_
 }
 
 void launch_cg_mask_dot(int64_t n, const signed char* mask, const double* p, double* q, double* partial, int nb,
-                        double* scal, hipStream_t s) {
+                        hipStream_t s) {
     hipLaunchKernelGGL(k_cg_mask_dot, dim3(nb), dim3(kDotThreads), 0, s, n, mask, p, q, partial);
-    hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(kDotThreads), 0, s, nb, partial, scal, 0);
 }
 
-void launch_cg_update_dot(int64_t n, double* scal, const double* p, const double* q, double* x, double* r,
-                          const double* pa, const double* pb, double* z, double* partial, int nb, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_update_dot, dim3(nb), dim3(kDotThreads), 0, s, n, scal, p, q, x, r, pa, pb, z, partial);
-    hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(kDotThreads), 0, s, nb, partial, scal, 1);
+void launch_cg_update_dot(int64_t n, const double* rz_new, const double* pq_partial, int npq, const double* p,
+                          const double* q, double* x, double* r, const double* pa, const double* pb, double* z,
+                          double* rz_partial, double* rr_partial, int nb, hipStream_t s) {
+    if (rr_partial)
+        hipLaunchKernelGGL(k_cg_update_dot<true>, dim3(nb), dim3(kDotThreads), 0, s, n, rz_new, pq_partial, npq, p, q,
+                           x, r, pa, pb, z, rz_partial, rr_partial);
+    else
+        hipLaunchKernelGGL(k_cg_update_dot<false>, dim3(nb), dim3(kDotThreads), 0, s, n, rz_new, pq_partial, npq, p, q,
+                           x, r, pa, pb, z, rz_partial, rr_partial);
+}
+
+void launch_dot_partials(int64_t n, const double* x, const double* y, double* partial, int nblocks, hipStream_t s) {
+    hipLaunchKernelGGL(k_dot_partial, dim3(nblocks), dim3(kDotThreads), 0, s, n, x, y, partial);
 }
 
 int dot_blocks(int64_t n) {
@@ -356,19 +372,12 @@ void launch_block_jacobi(int64_t n, const signed char* mask, const double* diag,
     if (n) hipLaunchKernelGGL(k_block_jacobi, grid1((n + 1) / 2), dim3(256), 0, s, n, mask, diag, offd, pa, pb);
 }
 
-void launch_cg_mask(int64_t n, const signed char* mask, double* q, hipStream_t s) {
-    if (n) hipLaunchKernelGGL(k_cg_mask, grid1(n), dim3(256), 0, s, n, mask, q);
+void launch_cg_direction(int64_t n, const double* rz_old, double* rz_new, const double* rz_partial, int nrz,
+                         const double* z, double* p, hipStream_t s) {
+    if (n)
+        hipLaunchKernelGGL(k_cg_direction, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)), dim3(kDotThreads),
+                           0, s, n, rz_old, rz_new, rz_partial, nrz, z, p);
 }
-
-void launch_cg_update(int64_t n, const double* scal, const double* p, const double* q, double* x, double* r,
-                      const double* pa, const double* pb, double* z, hipStream_t s) {
-    if (n) hipLaunchKernelGGL(k_cg_update, grid1((n + 1) / 2), dim3(256), 0, s, n, scal, p, q, x, r, pa, pb, z);
-}
-
-void launch_cg_direction(int64_t n, const double* scal, const double* z, double* p, hipStream_t s) {
-    if (n) hipLaunchKernelGGL(k_cg_direction, grid1(n), dim3(256), 0, s, n, scal, z, p);
-}
-
 
 void launch_axpy(int64_t n, double a, const double* x, double* y, hipStream_t s) {
     if (n) hipLaunchKernelGGL(k_axpy, grid1(n), dim3(256), 0, s, n, a, x, y);
