@@ -471,9 +471,10 @@ void release_data(ipf_ctx* ctx) {
 // 106 -> 100; Q3 2.56 M 159 -> 154.  Per CG iteration (nine launches -> three):
 // Q2 14 k 23.8 -> 12.9, 90 k 29.1 -> 16.8, 1.44 M 100.6 -> 85.1, 2.7 M 152 ->
 // 144, 5.8 M 280 -> 315.  Per product: 90 k 17.1 -> 9.0, 810 k 35.3 -> 32.1,
-// 2.7 M 87.9 -> 90.1; right after a residual and tangent (cold caches) 1.44 M
+// 2.7 M 87.9 -> 90.1.  Per residual with tangent: Q2 90 k 42.3 -> 19.5,
+// 1.44 M 149 -> 142, 2.7 M 239 -> 243; Q1 2.56 M 197 -> 207.  Products right after a residual and tangent (cold caches) 1.44 M
 // points already lose 2 us.
-constexpr int64_t kSplitPoints = 2500000, kSplitPointsProduct = 1000000;
+constexpr int64_t kSplitPoints = 2000000, kSplitPointsProduct = 1000000;
 
 // Whether the CG takes the element / node launches (three per iteration).
 bool cg_split(const ipf_ctx* ctx) {
@@ -482,12 +483,22 @@ bool cg_split(const ipf_ctx* ctx) {
 
 constexpr int kScal = 16;  // CG / Newton scalars in dScal
 
+// The B format of the residual with tangent: the geometric or the compact
+// FP64 values, or (neither at hand) the stored dense blocks, which take the
+// separate strain, stress and force launches.
+int dep_format(const ipf_ctx* ctx) {
+    return ctx->have_geometry ? FMT_G64 : ctx->dBf[FMT_C64] ? FMT_C64 : FMT_D64;
+}
+
 // Solver workspace, allocated once per transferred data set.
 int ensure_solver_buffers(ipf_ctx* ctx) {
-    if (ctx->dDep) return IPF_OK;
     int rc;
-    if ((rc = dev_alloc(ctx, &ctx->dDep, 9 * ctx->npad)) || (rc = dev_alloc(ctx, &ctx->dStrain, 3 * ctx->npts)) ||
-        (rc = dev_alloc(ctx, &ctx->dSigw, 3 * ctx->npts)) || (rc = dev_alloc(ctx, &ctx->dDiag, ctx->neq)) ||
+    if (dep_format(ctx) == FMT_D64 && !ctx->dSigw) {  // strains and stresses of the separate launches
+        if (!ctx->dStrain && (rc = dev_alloc(ctx, &ctx->dStrain, 3 * ctx->npts))) return rc;
+        if ((rc = dev_alloc(ctx, &ctx->dSigw, 3 * ctx->npts))) return rc;
+    }
+    if (ctx->dDep) return IPF_OK;
+    if ((rc = dev_alloc(ctx, &ctx->dDep, 9 * ctx->npad)) || (rc = dev_alloc(ctx, &ctx->dDiag, ctx->neq)) ||
         (rc = dev_alloc(ctx, &ctx->dOffd, ctx->neq)) || (rc = dev_alloc(ctx, &ctx->dPa, ctx->neq)) ||
         (rc = dev_alloc(ctx, &ctx->dPb, ctx->neq)) ||
         (rc = dev_alloc(ctx, &ctx->dCr, ctx->neq)) || (rc = dev_alloc(ctx, &ctx->dCz, ctx->neq)) ||
@@ -2016,6 +2027,7 @@ int ipf_point_features(ipf_ctx* ctx, const double* u_dev, float* feat_dev, int* 
         return fail(ctx, IPF_EINVAL, "ipf_point_features: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if ((rc = ensure_solver_buffers(ctx))) return rc;
+    if (!ctx->dStrain && (rc = dev_alloc(ctx, &ctx->dStrain, 3 * ctx->npts))) return rc;
     for (const auto& g : ctx->groups)
         launch_multiply(g.shape, group_dev(ctx, g), u_dev, ctx->dStrain, ctx->dOrig, ctx->stream);
     for (const auto& g : ctx->groups)
@@ -2222,9 +2234,34 @@ int ipf_set_dirichlet_mask(ipf_ctx* ctx, const signed char* mask_host) {
 
 namespace {
 
-// The launches of ipf_residual_tangent on stream s: strains, stresses with
-// w Dep, r = f_lin - B^T (w sigma).
-void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStream_t s) {
+// The launches of ipf_residual_tangent on stream s: r = f_lin - B^T (w sigma)
+// and w Dep, fused per element launch (split: dEf is free to use) or color.
+// Against strain, stress and force launches over the dense blocks (kept where
+// only those are stored), neither the dense B (432 bytes per point, twice) nor
+// the strains and stresses are read or written: with one product K v,
+// 1.44 M Q2 points 394 -> 167 us.
+void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStream_t s, bool split) {
+    const int fmt = dep_format(ctx);
+    if (split && fmt == FMT_G64 && !ctx->update_mem) {
+        const PointState st = point_state(ctx);
+        for (int sh = 0; sh < SHAPE_COUNT; sh++)
+            launch_elem_dep(sh, split_dev(ctx, sh), u, st, ctx->dDep, ctx->npad, ctx->dEf, s);
+        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, ctx->dFlin, r, s);
+        return;
+    }
+    if (fmt != FMT_D64) {
+        const double* flin = ctx->fold_flin ? ctx->dFlin : nullptr;
+        if (!flin) launch_copy(ctx->neq, ctx->dFlin, r, s);
+        const PointState st = point_state(ctx);
+        for (const auto& g : ctx->groups) {
+            GroupDev d = group_dev(ctx, g);
+            if (flin) d.dof = ctx->dDofR + g.dof_off;
+            if (ctx->dNodeR) d.node = ctx->dNodeR + g.dof_off / 2;
+            launch_residual_dep(fmt, g.shape, ctx->update_mem, d, group_fmt_B(ctx, g, fmt), u, r, flin, st, ctx->dDep,
+                                ctx->npad, s);
+        }
+        return;
+    }
     for (const auto& g : ctx->groups)
         launch_multiply(g.shape, group_dev(ctx, g), u, ctx->dStrain, ctx->dOrig, s);
     for (const auto& g : ctx->groups)
@@ -2297,7 +2334,7 @@ hipGraphExec_t newton_step_graph(ipf_ctx* ctx, const double* u) {
         (void)hipGetLastError();
         return nullptr;
     }
-    residual_tangent_launches(ctx, u, ctx->dNr, s);
+    residual_tangent_launches(ctx, u, ctx->dNr, s, cg_split(ctx));
     if (ctx->tfmt == FMT_G32) launch_to_f32(9 * ctx->npad, ctx->dDep, ctx->dDep32, s);
     masked_norm_launch(ctx, ctx->dNr, s);
     cg_start(ctx, ctx->dNr, ctx->dNd, 7, s);
@@ -2324,7 +2361,8 @@ int ipf_residual_tangent(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     if (!u_dev || !r_dev) return fail(ctx, IPF_EINVAL, "ipf_residual_tangent: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if ((rc = ensure_solver_buffers(ctx))) return rc;
-    residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream);
+    residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream,
+                              ctx->have_geometry && ctx->npad <= kSplitPoints && split_stream(ctx));
     ctx->have_tangent = true;
     ctx->dep32_ok = false;
     if ((rc = ensure_dep32(ctx))) return rc;

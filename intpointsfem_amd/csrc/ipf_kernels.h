@@ -190,6 +190,9 @@ void launch_pattern_positions(int shape, const GroupDev& g, const int64_t* ia, c
 // (certified_elastic, ipf_pointmath.h); ignored when commit is set.
 void launch_residual_fmt(int fmt, int shape, bool commit, bool fast, const GroupDev& g, const void* Bv,
                          const double* u, double* r, const double* flin, const PointState& st, hipStream_t stream);
+// The residual of one group with every point's w Dep (FMT_G64, FMT_C64).
+void launch_residual_dep(int fmt, int shape, bool commit, const GroupDev& g, const void* Bv, const double* u, double* r,
+                         const double* flin, const PointState& st, double* dep, int64_t npad, hipStream_t stream);
 // The tangent launches accumulate y += B^T (w Dep) B v; with zero_first,
 // g.dof's (g.node's) entries flagged kFirstWrite start from 0 instead of y[d],
 // so the launches of all groups overwrite y with K v and need no clear.

@@ -42,11 +42,15 @@ namespace {
 // certified_elastic takes its trial stress and skips the spectral
 // decomposition; a wavefront whose points all pass skips the return map's
 // instructions altogether.  The other points take the exact return map.
-template <int SHAPE, int FMT, bool COMMIT, bool PAIR, bool FAST>
-__global__ void __launch_bounds__(kWave, (FC<SHAPE, FMT>::MIN_WAVES))
+//
+// DEP: the residual with every point's consistent tangent, w Dep to dep (SoA,
+// npad apart): one launch per color in place of strain, stress and force
+// launches over the stored dense B.
+template <int SHAPE, int FMT, bool COMMIT, bool PAIR, bool FAST, bool DEP = false>
+__global__ void __launch_bounds__(kWave, (DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
 k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict__ u, double* __restrict__ r,
-               const double* __restrict__ flin, PointState st) {
-    static_assert(!(FAST && COMMIT), "the certified elastic path commits nothing");
+               const double* __restrict__ flin, PointState st, double* __restrict__ dep, int64_t npad) {
+    static_assert(!(FAST && (COMMIT || DEP)), "the certified elastic path commits nothing and has no tangent");
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
     constexpr int NSH = C::CE / 2;
@@ -151,7 +155,14 @@ k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict
         int mt, br;
         const double w = FmtTraits<FMT>::GEOM ? wgeo : wst;
         const MatConst& mc = tile_material(g, tile);
-        if (!(FAST && certified_elastic(e3, ep, mc, w, ws))) point_sigma<false>(e3, ep, alpha, mt, br, mc, w, ws, nullptr);
+        if constexpr (DEP) {
+            double d9[9];
+            point_sigma<true>(e3, ep, alpha, mt, br, mc, w, ws, d9);
+#pragma unroll
+            for (int k = 0; k < 9; k++) dep[k * npad + P] = d9[k];
+        } else if (!(FAST && certified_elastic(e3, ep, mc, w, ws))) {
+            point_sigma<false>(e3, ep, alpha, mt, br, mc, w, ws, nullptr);
+        }
         if (COMMIT) {
             st.ep0[P] = ep[0];
             st.ep1[P] = ep[1];
@@ -553,15 +564,33 @@ void residual_fmt_shape(bool commit, bool fast, const GroupDev& g, const void* B
                         const double* flin, const PointState& st, hipStream_t s) {
     const dim3 grid((unsigned)g.ntiles), block(kWave);
     if (commit)
-        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, true, false, false>), grid, block, 0, s, g, Bv, u, r, flin, st);
+        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, true, false, false>), grid, block, 0, s, g, Bv, u, r, flin, st, nullptr, (int64_t)0);
     else if (g.node && fast)
-        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, true, true>), grid, block, 0, s, g, Bv, u, r, flin, st);
+        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, true, true>), grid, block, 0, s, g, Bv, u, r, flin, st, nullptr, (int64_t)0);
     else if (g.node)
-        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, true, false>), grid, block, 0, s, g, Bv, u, r, flin, st);
+        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, true, false>), grid, block, 0, s, g, Bv, u, r, flin, st, nullptr, (int64_t)0);
     else if (fast)
-        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, false, true>), grid, block, 0, s, g, Bv, u, r, flin, st);
+        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, false, true>), grid, block, 0, s, g, Bv, u, r, flin, st, nullptr, (int64_t)0);
     else
-        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, false, false>), grid, block, 0, s, g, Bv, u, r, flin, st);
+        hipLaunchKernelGGL((k_residual_fmt<SHAPE, FMT, false, false, false>), grid, block, 0, s, g, Bv, u, r, flin, st, nullptr, (int64_t)0);
+}
+
+template <int FMT>
+void residual_dep(int shape, bool commit, const GroupDev& g, const void* Bv, const double* u, double* r,
+                  const double* flin, const PointState& st, double* dep, int64_t npad, hipStream_t s) {
+    const dim3 grid((unsigned)g.ntiles), block(kWave);
+    dispatch_shape(shape, [&](auto sc) {
+        constexpr int S = decltype(sc)::value;
+        if (commit)
+            hipLaunchKernelGGL((k_residual_fmt<S, FMT, true, false, false, true>), grid, block, 0, s, g, Bv, u, r, flin,
+                               st, dep, npad);
+        else if (g.node)
+            hipLaunchKernelGGL((k_residual_fmt<S, FMT, false, true, false, true>), grid, block, 0, s, g, Bv, u, r, flin,
+                               st, dep, npad);
+        else
+            hipLaunchKernelGGL((k_residual_fmt<S, FMT, false, false, false, true>), grid, block, 0, s, g, Bv, u, r,
+                               flin, st, dep, npad);
+    });
 }
 
 template <int FMT>
@@ -614,6 +643,15 @@ void launch_residual_fmt(int fmt, int shape, bool commit, bool fast, const Group
         case FMT_C32: residual_fmt<FMT_C32>(shape, commit, f, g, Bv, u, r, flin, st, s); break;
         default: break;
     }
+}
+
+void launch_residual_dep(int fmt, int shape, bool commit, const GroupDev& g, const void* Bv, const double* u, double* r,
+                         const double* flin, const PointState& st, double* dep, int64_t npad, hipStream_t s) {
+    if (g.ntiles == 0) return;
+    if (fmt == FMT_G64)
+        residual_dep<FMT_G64>(shape, commit, g, Bv, u, r, flin, st, dep, npad, s);
+    else if (fmt == FMT_C64)
+        residual_dep<FMT_C64>(shape, commit, g, Bv, u, r, flin, st, dep, npad, s);
 }
 
 void launch_tangent_fmt(int fmt, int shape, const GroupDev& g, const void* Bv, const double* v, double* y,

@@ -31,6 +31,9 @@ struct SplitDev {
 // ef[entry] (two doubles) = the element's force on its node, fmt FMT_G64 / FMT_G32
 void launch_elem_residual(int fmt, int shape, bool fast, const SplitDev& g, const double* u, const PointState& st,
                           double* ef, hipStream_t stream);
+// The residual's element forces and every point's w Dep (FMT_G64).
+void launch_elem_dep(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, int64_t npad,
+                     double* ef, hipStream_t stream);
 // With rz_old (a CG iteration, see ipf_kernels.h): v is z, and the vector
 // multiplied is z + beta p, formed as it is gathered.
 struct CgBeta {
@@ -39,7 +42,7 @@ struct CgBeta {
     const double* rz_partial;
     int nrz;
 };
-void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, const double* dep,
+void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, double* dep,
                          const float* dep32, int64_t npad, double* ef, hipStream_t stream);
 
 // map: stride (4 or 8) ints per node, one per color; filled with -1, then one

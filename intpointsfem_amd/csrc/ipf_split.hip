@@ -15,7 +15,7 @@ namespace ipf {
 
 namespace {
 
-enum ElemOp { EL_RESIDUAL = 0, EL_CERTIFIED = 1, EL_TANGENT = 2, EL_CG = 3 };
+enum ElemOp { EL_RESIDUAL = 0, EL_CERTIFIED = 1, EL_TANGENT = 2, EL_CG = 3, EL_DEP = 4 };
 
 // One wavefront per tile: gather, strain, stress (or w Dep times the strain),
 // B^T products and the sums over each element's points, as k_residual_fmt /
@@ -26,8 +26,8 @@ enum ElemOp { EL_RESIDUAL = 0, EL_CERTIFIED = 1, EL_TANGENT = 2, EL_CG = 3 };
 // and last round trip (a product with w Dep requested after the gather and
 // the addresses read from a table: 20x20 Q2 7.8 us, so 6.3).
 template <int SHAPE, int FMT, int OP>
-__global__ void __launch_bounds__(kWave, (FC<SHAPE, FMT>::MIN_WAVES))
-k_elem(SplitDev g, const double* __restrict__ u, PointState st, const double* __restrict__ dep,
+__global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
+k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restrict__ dep,
        const float* __restrict__ dep32, int64_t npad, CgBeta cg, dv2* __restrict__ ef) {
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
@@ -121,7 +121,13 @@ k_elem(SplitDev g, const double* __restrict__ u, PointState st, const double* __
             }
         } else {
             const MatConst& mc = g.mats[tm >> 8];
-            if (!(OP == EL_CERTIFIED && certified_elastic(e3, ep, mc, w, x))) {
+            if constexpr (OP == EL_DEP) {
+                double alpha = 0.0, d9[9];
+                int mt, br;
+                point_sigma<true>(e3, ep, alpha, mt, br, mc, w, x, d9);
+#pragma unroll
+                for (int k = 0; k < 9; k++) dep[k * npad + P] = d9[k];
+            } else if (!(OP == EL_CERTIFIED && certified_elastic(e3, ep, mc, w, x))) {
                 double alpha = 0.0;
                 int mt, br;
                 point_sigma<false>(e3, ep, alpha, mt, br, mc, w, x, nullptr);
@@ -276,7 +282,7 @@ k_nodes_cg(int64_t n, const int* __restrict__ map, const dv2* __restrict__ ef, c
 }
 
 template <int FMT, int OP>
-void elem(int shape, const SplitDev& g, const double* u, const PointState& st, const double* dep, const float* dep32,
+void elem(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, const float* dep32,
           int64_t npad, const CgBeta& cg, double* ef, hipStream_t s) {
     dispatch_shape(shape, [&](auto sc) {
         constexpr int S = decltype(sc)::value;
@@ -303,7 +309,12 @@ void launch_elem_residual(int fmt, int shape, bool fast, const SplitDev& g, cons
     }
 }
 
-void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, const double* dep,
+void launch_elem_dep(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, int64_t npad,
+                     double* ef, hipStream_t s) {
+    if (g.ntiles) elem<FMT_G64, EL_DEP>(shape, g, u, st, dep, nullptr, npad, CgBeta{}, ef, s);
+}
+
+void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, double* dep,
                          const float* dep32, int64_t npad, double* ef, hipStream_t s) {
     if (g.ntiles == 0) return;
     const PointState none{};

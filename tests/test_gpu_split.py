@@ -1,7 +1,7 @@
 """The element / node launches against the launch per color.
 
-Bars: residual and tangent product bit-identical (the node launch sums in
-color order), on meshes from one element up, every order, uneven batches with
+Bars: residual, residual with tangent and tangent product bit-identical (the
+node launch sums in color order), on meshes from one element up, every order, uneven batches with
 several materials and triangles next to quadrilaterals; a CG solution's own
 residual ||b - K x|| <= 10 rtol ||b|| (the recurrence's residual is <= rtol
 ||b||; the true one may drift from it by rounding).  A second stream keeps the
@@ -47,7 +47,25 @@ def compare(gpu, ctx, u, v):
         ctx.set_residual_mode(mode)
         a, b = both_ways(gpu, ctx, neq, lambda out: ctx.residual(du, out))
         assert np.isfinite(a).all() and np.array_equal(a, b), mode
-    ctx.residual_tangent(du, torch.zeros_like(du))
+    kv = []
+
+    def tangent(out):
+        y = torch.zeros_like(out)
+        ctx.residual_tangent(du, out)
+        ctx.tangent_apply(dv, y)
+        kv.append(y)
+    r, s = both_ways(gpu, ctx, neq, tangent)
+    assert np.array_equal(r, s) and torch.equal(kv[0], kv[1])
+    # committing, the residual with tangent leaves the state the residual leaves
+    before, states = ctx.get_state(), []
+    for call in (ctx.residual, ctx.residual_tangent):
+        ctx.set_state(before[0], before[1])
+        ctx.set_update_mem(True)
+        call(du, torch.zeros_like(du))
+        ctx.set_update_mem(False)
+        states.append(ctx.get_state())
+    assert all(np.array_equal(x, y) for x, y in zip(*states))
+    ctx.set_state(before[0], before[1])
     for fmt in ("geometry-fp64", "geometry-fp32"):
         ctx.set_b_format("geometry-fp64", fmt)
         a, b = both_ways(gpu, ctx, neq, lambda out: ctx.tangent_apply(dv, out))
