@@ -320,6 +320,9 @@ struct ipf_ctx {
     int* dLidx = nullptr;
     int64_t nnz_k = 0;
     bool have_pattern = false;
+    // every CSR entry has an element: its first one in launch order (flagged
+    // kFirstWrite in dLidx) starts it from 0, and Kg needs no clear
+    bool fold_kg = false;
     // the pattern itself when ipf_build_tangent_pattern built it on the device
     int64_t* dPatIA = nullptr;  // [neq + 1]
     int64_t* dPatJA = nullptr;  // [nnz_k]
@@ -2421,12 +2424,33 @@ int ipf_set_tangent_pattern(ipf_ctx* ctx, const int* el_color_index, const int64
         }
         off += nt;
     }
+    // first elements of the entries, in launch order
+    int64_t touched = 0;
+    try {
+        std::vector<char> has(nnz, 0);
+        for (const auto& g : ctx->groups) {
+            const int64_t ce = shape_ce(g.shape), nt = ce * (ce + 1) / 2;
+            for (size_t k = 0; k < g.elems.size(); k++) {
+                if (g.elems[k] < 0) continue;
+                int* p = L.data() + g.l_off + (int64_t)k * nt;
+                for (int64_t t = 0; t < nt; t++)
+                    if (!has[p[t]]) {
+                        has[p[t]] = 1;
+                        touched++;
+                        p[t] |= kFirstWrite;
+                    }
+            }
+        }
+    } catch (const std::bad_alloc&) {
+        return fail(ctx, IPF_EINVAL, "ipf_set_tangent_pattern: host allocation failed");
+    }
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     dev_free(ctx->dLidx);
     dev_free(ctx->dPatIA);
     dev_free(ctx->dPatJA);
     ctx->have_pattern = false;
+    ctx->fold_kg = touched == nnz;
     if ((rc = dev_alloc(ctx, &ctx->dLidx, total))) return rc;
     if (total) IPF_HIP(ctx, hipMemcpy(ctx->dLidx, L.data(), sizeof(int) * (size_t)total, hipMemcpyHostToDevice));
     ctx->nnz_k = nnz;
@@ -2490,13 +2514,18 @@ int ipf_build_tangent_pattern(ipf_ctx* ctx, int64_t* nnz) {
     launch_pattern_rows(keys, n, ctx->neq, ctx->dPatIA, ctx->dPatJA, s);
     for (const auto& g : ctx->groups)
         launch_pattern_positions(g.shape, group_dev(ctx, g), ctx->dPatIA, ctx->dPatJA, ctx->dLidx + g.l_off, s);
-    e = hipGetLastError();
+    // every entry comes from an element; keys (8 bytes per element entry, at
+    // least as many as entries) holds the marks now
+    e = hipMemsetAsync(keys, 0, (size_t)n, s);
+    for (const auto& g : ctx->groups)
+        launch_pattern_first(g.shape, group_dev(ctx, g), ctx->dLidx + g.l_off, reinterpret_cast<signed char*>(keys), s);
+    if (e == hipSuccess) e = hipGetLastError();
     const hipError_t e2 = hipStreamSynchronize(s);
     dev_free(keys);
     if (e != hipSuccess || e2 != hipSuccess)
         return fail(ctx, IPF_EHIP, "ipf_build_tangent_pattern: %s", hipGetErrorString(e != hipSuccess ? e : e2));
     ctx->nnz_k = n;
-    ctx->have_pattern = true;
+    ctx->have_pattern = ctx->fold_kg = true;
     *nnz = n;
     return IPF_OK;
 }
@@ -2517,10 +2546,10 @@ int ipf_assemble_tangent(ipf_ctx* ctx, const double* u_dev, double* r_dev, doubl
     if (!kg_dev) return fail(ctx, IPF_EINVAL, "ipf_assemble_tangent: NULL pointer");
     if (!ctx->have_pattern) return fail(ctx, IPF_ESTATE, "no tangent pattern: call ipf_set_tangent_pattern first");
     if ((rc = ipf_residual_tangent(ctx, u_dev, r_dev))) return rc;
-    launch_fill(ctx->nnz_k, kg_dev, 0.0, ctx->stream);
+    if (!ctx->fold_kg) launch_fill(ctx->nnz_k, kg_dev, 0.0, ctx->stream);
     for (const auto& g : ctx->groups)
-        launch_assemble_K(g.shape, group_dev(ctx, g), ctx->dDep, ctx->npad, ctx->dLidx + g.l_off, kg_dev,
-                          ctx->stream);
+        launch_assemble_K(g.shape, group_dev(ctx, g), ctx->have_geometry ? ctx->dGeo + 8 * g.slot0 : nullptr,
+                          ctx->compact_ok, ctx->dDep, ctx->npad, ctx->dLidx + g.l_off, kg_dev, ctx->stream);
     return launch_status(ctx, "assemble_tangent");
 }
 

@@ -162,9 +162,11 @@ void launch_tangent_diag(int shape, const GroupDev& g, double* diag, double* off
 
 // Tangent stiffness into CSR values (ipf_assemble.hip): kg[lidx[e * NT + t]] +=
 // entry t of element e's packed upper triangle (NT = CE (CE + 1) / 2), for
-// the elements of one group (B: the dense FP64 tiles).
-void launch_assemble_K(int shape, const GroupDev& g, const double* dep_soa, int64_t npad, const int* lidx,
-                       double* kg, hipStream_t stream);
+// the elements of one group (B: the dense FP64 tiles).  A position flagged
+// kFirstWrite starts from 0.  pattern: every block has the 2D elasticity
+// pattern (dN_a/dx, dN_a/dy); geo (or null): the group's corners.
+void launch_assemble_K(int shape, const GroupDev& g, const double* geo, bool pattern, const double* dep_soa,
+                       int64_t npad, const int* lidx, double* kg, hipStream_t stream);
 
 // The tangent's CSR pattern on the device (ipf_pattern.hip): keys of a
 // group's element entries (packed upper triangles by element slot, like
@@ -178,6 +180,9 @@ void launch_pattern_rows(const uint64_t* uniq, int64_t nnz, int64_t neq, int64_t
                          hipStream_t stream);
 void launch_pattern_positions(int shape, const GroupDev& g, const int64_t* ia, const int64_t* ja, int* lidx,
                               hipStream_t stream);
+// kFirstWrite on the group's positions not seen yet; marks them seen (groups
+// in launch order; a group's elements share no position)
+void launch_pattern_first(int shape, const GroupDev& g, int* lidx, signed char* seen, hipStream_t stream);
 
 // The fused residual and the tangent product (ipf_kernels_fmt.hip): Bv points
 // at the group's first tile in format fmt (FMT_D64: the dense tiles g.B;

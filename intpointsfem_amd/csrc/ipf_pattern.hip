@@ -99,7 +99,29 @@ __global__ void k_pattern_positions(GroupDev g, const int64_t* __restrict__ ia, 
     }
 }
 
+template <int SHAPE>
+__global__ void k_pattern_first(GroupDev g, int* __restrict__ lidx, signed char* __restrict__ seen) {
+    constexpr int CE = shape_ce(SHAPE), NT = CE * (CE + 1) / 2, ET = shape_et(SHAPE);
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= g.nelem * NT) return;
+    const int64_t slot = i / NT;
+    if ((int)(slot % ET) >= tile_nvalid(g, slot / ET)) return;
+    const int l = lidx[i];
+    if (seen[l]) return;
+    seen[l] = 1;
+    lidx[i] = l | kFirstWrite;
+}
+
 }  // namespace
+
+void launch_pattern_first(int shape, const GroupDev& g, int* lidx, signed char* seen, hipStream_t s) {
+    const int64_t n = g.nelem * (shape_ce(shape) * (shape_ce(shape) + 1) / 2);
+    if (n == 0) return;
+    const dim3 grid((unsigned)((n + kBlock - 1) / kBlock)), block(kBlock);
+    dispatch_shape(shape, [&](auto sc) {
+        hipLaunchKernelGGL((k_pattern_first<decltype(sc)::value>), grid, block, 0, s, g, lidx, seen);
+    });
+}
 
 void launch_pattern_keys(int shape, const GroupDev& g, int64_t neq, uint64_t* keys, hipStream_t s) {
     const int64_t n = g.nelem * shape_ce(shape);
