@@ -309,8 +309,9 @@ enum {
 /* Selects the B representation of the fused residual (ipf_residual,
  * ipf_residual_timed, and the commit inside ipf_newton) and, separately, of
  * the tangent product (ipf_tangent_apply and the CG matvecs).  The
- * separate-step entry points and ipf_residual_tangent keep the dense FP64
- * blocks.  The compact forms hold only dN_a/dx and dN_a/dy per point -- the
+ * separate-step entry points and ipf_residual_tangent form B in FP64 from the
+ * corners or the compact values where either is at hand, and read the dense
+ * FP64 blocks elsewhere (the same results).  The compact forms hold only dN_a/dx and dN_a/dy per point -- the
  * reference's blocks carry nothing else (TPZNumericalIntegrator.cpp:371-381);
  * ipf_transfer_data checks that pattern exactly and this call fails with
  * IPF_EINVAL when it does not hold.  Compact FP64 gives the dense FP64

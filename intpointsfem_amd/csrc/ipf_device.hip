@@ -73,6 +73,10 @@ MatConst MatConst::make(double lambda, double mu, double mc_phi, double mc_psi, 
     const double cotphi = 1. / tan(mc_phi);
     m.c_cot = c * cotphi;
     m.apex_alpha = cos(mc_phi) / sin(mc_psi);
+    m.feat_c = m.phi_c / (2. * cosphi);
+    m.feat_lnc = (float)log(m.feat_c);
+    m.feat_phi = (float)asin(sinphi);
+    m.feat_psi = (float)asin(sinpsi);
     // principal-space tangents, FunctionsSigmaProjection.h:68-88, :163-188, :262-287
     {
         const double sin_phi = sinphi, sin_psi = sinpsi;
@@ -392,6 +396,7 @@ void release_patch(ipf_ctx* ctx) {
 void release_split(ipf_ctx* ctx) {
     dev_free(ctx->dMap);
     dev_free(ctx->dEf);
+    for (auto& d : ctx->split) d = SplitDev{};
     ctx->split_ok = false;
     ctx->ef_bound = false;
 }
@@ -479,9 +484,14 @@ void release_data(ipf_ctx* ctx) {
 // points already lose 2 us.
 constexpr int64_t kSplitPoints = 2000000, kSplitPointsProduct = 1000000;
 
+// The B formats of the element launches: geometric or compact FP64.
+bool split_format(const ipf_ctx* ctx, int fmt) {
+    return format_geometric(fmt) ? ctx->have_geometry : fmt == FMT_C64 && ctx->dBf[FMT_C64];
+}
+
 // Whether the CG takes the element / node launches (three per iteration).
 bool cg_split(const ipf_ctx* ctx) {
-    return ctx->split_ok && ctx->npad <= kSplitPoints && format_geometric(ctx->tfmt);
+    return ctx->split_ok && ctx->npad <= kSplitPoints && split_format(ctx, ctx->tfmt);
 }
 
 constexpr int kScal = 16;  // CG / Newton scalars in dScal
@@ -736,9 +746,10 @@ const double* residual_start(ipf_ctx* ctx, double* r) {
     return nullptr;
 }
 
-// The launches and the node map of the element / node launches: geometric
-// data whose elements number their nodes' DoFs as aligned (x, y) pairs, in at
-// most 8 colors.  Out of memory leaves the colored launches (not an error).
+// The element launches of every shape (segments of at most 8 colors) and, for
+// elements that number their nodes' DoFs as aligned (x, y) pairs, the node map
+// of the element / node launches.  Out of memory leaves the colored launches
+// (not an error).
 void build_split(ipf_ctx* ctx) {
     const int stride = ctx->ncolor <= 4 ? 4 : 8;
     int64_t nent = 0, ntile = 0;
@@ -746,13 +757,11 @@ void build_split(ipf_ctx* ctx) {
         nent = std::max(nent, g.dof_off / 2 + (int64_t)g.elems.size() * (shape_ce(g.shape) / 2));
         ntile += g.ntiles;
     }
-    if (!ctx->have_geometry || !ctx->pairs_aligned || ctx->ncolor > kSplitColors || ntile == 0 || nent > INT32_MAX ||
-        ctx->npad > INT32_MAX)
+    if (!ctx->pairs_aligned || ctx->ncolor > kSplitColors || ntile == 0 || nent > INT32_MAX || ctx->npad > INT32_MAX)
         return;
     for (int sh = 0; sh < SHAPE_COUNT; sh++) {
         SplitDev& d = ctx->split[sh];
         d = SplitDev{};
-        if (ctx->tab_off[sh] < 0) continue;
         const int ET = shape_et(sh), NE = ET * (shape_ce(sh) / 2), TP = shape_tp(sh);
         for (const auto& g : ctx->groups) {
             if (g.shape != sh) continue;
@@ -761,12 +770,11 @@ void build_split(ipf_ctx* ctx) {
             d.pt0[d.nseg] = (int)(g.pt0 - t0 * TP);
             d.slot0[d.nseg] = (int)(g.slot0 - t0 * ET);
             d.ent0[d.nseg] = (int)(g.dof_off / 2 - t0 * NE);
+            d.val0[d.nseg] = g.f_off[FMT_C64] - t0 * format_values(sh, FMT_C64) * TP;
             d.ntiles += g.ntiles;
             d.end[d.nseg++] = (int)d.ntiles;
         }
         d.tmeta = ctx->dTmeta;
-        d.geo = ctx->dGeo;
-        d.tab = ctx->dTab + ctx->tab_off[sh];
         d.node = ctx->dNodeR;
     }
     const int64_t nnode = (ctx->neq + 1) / 2;
@@ -802,17 +810,61 @@ bool split_stream(ipf_ctx* ctx) {
     return true;
 }
 
-SplitDev split_dev(const ipf_ctx* ctx, int sh) {
-    SplitDev d = ctx->split[sh];
-    d.mats = ctx->dMats;  // replaced by ipf_set_material_table
-    return d;
+// The element launches of one operation over every shape, in B format fmt
+// (split_format).
+void elem_launches(ipf_ctx* ctx, int op, int fmt, const ElemArgs& a, hipStream_t s) {
+    for (int sh = 0; sh < SHAPE_COUNT; sh++) {
+        if (!ctx->split[sh].ntiles) continue;
+        SplitDev d = ctx->split[sh];
+        d.B = format_geometric(fmt) ? static_cast<const void*>(ctx->dGeo) : ctx->dBf[fmt];
+        d.tab = format_geometric(fmt) ? ctx->dTab + ctx->tab_off[sh] : nullptr;
+        d.mats = ctx->dMats;
+        launch_elem(op, fmt, sh, d, a, s);
+    }
 }
 
-// the element forces of K v into ef
-void elem_tangent(ipf_ctx* ctx, const double* v, const CgBeta& cg, double* ef, hipStream_t s) {
-    for (int sh = 0; sh < SHAPE_COUNT; sh++)
-        if (ctx->split[sh].ntiles)
-            launch_elem_tangent(ctx->tfmt, sh, split_dev(ctx, sh), v, cg, ctx->dDep, ctx->dDep32, ctx->npad, ef, s);
+// r = start - sum of the element forces ef (start null: 0)
+void node_launch(ipf_ctx* ctx, const double* ef, const double* start, double* r, hipStream_t s) {
+    launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ef, start, r, s);
+}
+
+ElemArgs elem_args(ipf_ctx* ctx, const double* u, double* ef) {
+    ElemArgs a{};
+    a.u = u;
+    a.st = point_state(ctx);
+    a.dep = ctx->dDep;
+    a.dep32 = ctx->dDep32;
+    a.npad = ctx->npad;
+    a.ef = ef;
+    a.orig = ctx->dOrig;
+    return a;
+}
+
+// Strains of u at every point (reference order).
+void strain_launches(ipf_ctx* ctx, const double* u, double* strain, hipStream_t s) {
+    if (ctx->split_ok && dep_format(ctx) != FMT_D64) {
+        ElemArgs a = elem_args(ctx, u, nullptr);
+        a.point = strain;
+        elem_launches(ctx, EL_STRAIN, dep_format(ctx), a, s);
+        return;
+    }
+    for (const auto& g : ctx->groups) launch_multiply(g.shape, group_dev(ctx, g), u, strain, ctx->dOrig, s);
+}
+
+// The return map from strains in the reference order.
+void stress_launches(ipf_ctx* ctx, const double* strain, double* wsigma, double* wdep) {
+    const PointState st = point_state(ctx);
+    if (ctx->split_ok) {
+        for (int sh = 0; sh < SHAPE_COUNT; sh++) {
+            SplitDev d = ctx->split[sh];
+            d.mats = ctx->dMats;
+            launch_stress(sh, d, strain, wsigma, wdep, ctx->dOrig, st, ctx->update_mem, ctx->stream);
+        }
+        return;
+    }
+    for (const auto& g : ctx->groups)
+        launch_sigma(wdep != nullptr, ctx->update_mem, g.shape, group_dev(ctx, g), ctx->npad, strain, wsigma, wdep,
+                     ctx->dOrig, st, ctx->stream);
 }
 
 // y = K v on stream s: the tangent launches of every group in the selected
@@ -869,10 +921,11 @@ void cg_iterations(ipf_ctx* ctx, double* x, int count, hipStream_t s) {
         double *pq = ctx->dPartial, *rz = ctx->dPartial + 1024;
         double* p = split && (k & 1) == 0 ? ctx->dCp2 : ctx->dCp;
         if (split) {
-            const CgBeta cg{(k & 1) == 0 ? ctx->dCp : ctx->dCp2, rz_old, rz, nb};
-            elem_tangent(ctx, ctx->dCz, cg, ctx->dEfS, s);
-            launch_nodes_cg(n, ctx->map_stride, ctx->dMap, ctx->dEfS, ctx->dMask, ctx->dCz, cg, rz_new, p, ctx->dCq, pq,
-                            nb, s);
+            ElemArgs a = elem_args(ctx, ctx->dCz, ctx->dEfS);
+            a.cg = CgBeta{(k & 1) == 0 ? ctx->dCp : ctx->dCp2, rz_old, rz, nb};
+            elem_launches(ctx, EL_CG, ctx->tfmt, a, s);
+            launch_nodes_cg(n, ctx->map_stride, ctx->dMap, ctx->dEfS, ctx->dMask, ctx->dCz, a.cg, rz_new, p, ctx->dCq,
+                            pq, nb, s);
         } else {
             launch_cg_direction(n, rz_old, rz_new, rz, nb, ctx->dCz, p, s);
             tangent_product(ctx, p, ctx->dCq, s);
@@ -1488,13 +1541,8 @@ static int transfer_impl(ipf_ctx* ctx, int64_t nblocks, const int* row_sizes, co
             release_data(ctx);
             return rc;
         }
-        ctx->have_geometry = true;
-        build_split(ctx);
-        if ((rc = launch_status(ctx, "node map"))) {
-            release_data(ctx);
-            return rc;
-        }
         IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        ctx->have_geometry = true;
     }
     ctx->have_data = true;
     ctx->patch_in = std::move(pin);
@@ -1507,6 +1555,14 @@ static int transfer_impl(ipf_ctx* ctx, int64_t nblocks, const int* row_sizes, co
     } else if (compact_ok) {
         if ((rc = ensure_format(ctx, FMT_C64))) return rc;
         ctx->rfmt = ctx->tfmt = FMT_C64;
+    }
+    if (geo || compact_ok) {
+        build_split(ctx);
+        if ((rc = launch_status(ctx, "node map"))) {
+            release_data(ctx);
+            return rc;
+        }
+        IPF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
     return IPF_OK;
 }
@@ -1894,13 +1950,10 @@ int ipf_residual(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     if (!u_dev || !r_dev) return fail(ctx, IPF_EINVAL, "ipf_residual: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if (ctx->assembly == IPF_ASSEMBLY_PATCH && !ctx->update_mem) return patch_residual(ctx, u_dev, r_dev);
-    if (!ctx->update_mem && format_geometric(ctx->rfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
-        const PointState st = point_state(ctx);
-        for (int sh = 0; sh < SHAPE_COUNT; sh++)
-            if (ctx->split[sh].ntiles)
-                launch_elem_residual(ctx->rfmt, sh, ctx->residual_mode == IPF_RESIDUAL_CERTIFIED_ELASTIC,
-                                     split_dev(ctx, sh), u_dev, st, ctx->dEf, ctx->stream);
-        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, ctx->dFlin, r_dev, ctx->stream);
+    if (!ctx->update_mem && split_format(ctx, ctx->rfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
+        elem_launches(ctx, ctx->residual_mode == IPF_RESIDUAL_CERTIFIED_ELASTIC ? EL_CERTIFIED : EL_RESIDUAL, ctx->rfmt,
+                      elem_args(ctx, u_dev, ctx->dEf), ctx->stream);
+        node_launch(ctx, ctx->dEf, ctx->dFlin, r_dev, ctx->stream);
         return launch_status(ctx, "residual");
     }
     // r = f_lin, then each color adds -B^T(w sigma)
@@ -1991,8 +2044,7 @@ int ipf_multiply(ipf_ctx* ctx, const double* u_dev, double* strain_dev) {
     if (rc) return rc;
     if (!u_dev || !strain_dev) return fail(ctx, IPF_EINVAL, "ipf_multiply: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    for (const auto& g : ctx->groups)
-        launch_multiply(g.shape, group_dev(ctx, g), u_dev, strain_dev, ctx->dOrig, ctx->stream);
+    strain_launches(ctx, u_dev, strain_dev, ctx->stream);
     return launch_status(ctx, "multiply");
 }
 
@@ -2017,9 +2069,7 @@ int ipf_compute_sigma(ipf_ctx* ctx, const double* strain_dev, double* wsigma_dev
     if (rc) return rc;
     if (!strain_dev || !wsigma_dev) return fail(ctx, IPF_EINVAL, "ipf_compute_sigma: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    for (const auto& g : ctx->groups)
-        launch_sigma(false, ctx->update_mem, g.shape, group_dev(ctx, g), ctx->npad, strain_dev, wsigma_dev, nullptr,
-                     ctx->dOrig, point_state(ctx), ctx->stream);
+    stress_launches(ctx, strain_dev, wsigma_dev, nullptr);
     return launch_status(ctx, "compute_sigma");
 }
 
@@ -2029,10 +2079,16 @@ int ipf_point_features(ipf_ctx* ctx, const double* u_dev, float* feat_dev, int* 
     if (!u_dev || !feat_dev || !branch_dev || !target_dev)
         return fail(ctx, IPF_EINVAL, "ipf_point_features: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if ((rc = ensure_solver_buffers(ctx))) return rc;
+    if (ctx->split_ok && dep_format(ctx) != FMT_D64) {
+        ElemArgs a = elem_args(ctx, u_dev, nullptr);
+        a.feat = feat_dev;
+        a.label = branch_dev;
+        a.target = target_dev;
+        elem_launches(ctx, EL_FEATURES, dep_format(ctx), a, ctx->stream);
+        return launch_status(ctx, "point_features");
+    }
     if (!ctx->dStrain && (rc = dev_alloc(ctx, &ctx->dStrain, 3 * ctx->npts))) return rc;
-    for (const auto& g : ctx->groups)
-        launch_multiply(g.shape, group_dev(ctx, g), u_dev, ctx->dStrain, ctx->dOrig, ctx->stream);
+    strain_launches(ctx, u_dev, ctx->dStrain, ctx->stream);
     for (const auto& g : ctx->groups)
         launch_point_features(g.shape, group_dev(ctx, g), ctx->dStrain, ctx->dOrig, point_state(ctx), feat_dev,
                               branch_dev, target_dev, ctx->stream);
@@ -2084,9 +2140,7 @@ int ipf_compute_sigma_dep(ipf_ctx* ctx, const double* strain_dev, double* wsigma
     if (rc) return rc;
     if (!strain_dev || !wsigma_dev || !wdep_dev) return fail(ctx, IPF_EINVAL, "ipf_compute_sigma_dep: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    for (const auto& g : ctx->groups)
-        launch_sigma(true, ctx->update_mem, g.shape, group_dev(ctx, g), ctx->npad, strain_dev, wsigma_dev, wdep_dev,
-                     ctx->dOrig, point_state(ctx), ctx->stream);
+    stress_launches(ctx, strain_dev, wsigma_dev, wdep_dev);
     return launch_status(ctx, "compute_sigma_dep");
 }
 
@@ -2095,6 +2149,13 @@ int ipf_multiply_transpose(ipf_ctx* ctx, const double* wsigma_dev, double* res_d
     if (rc) return rc;
     if (!wsigma_dev || !res_dev) return fail(ctx, IPF_EINVAL, "ipf_multiply_transpose: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
+    if (ctx->split_ok && dep_format(ctx) != FMT_D64 && split_stream(ctx)) {
+        ElemArgs a = elem_args(ctx, nullptr, ctx->dEf);
+        a.point = const_cast<double*>(wsigma_dev);  // read only
+        elem_launches(ctx, EL_FORCE, dep_format(ctx), a, ctx->stream);
+        node_launch(ctx, ctx->dEf, nullptr, res_dev, ctx->stream);
+        return launch_status(ctx, "multiply_transpose");
+    }
     launch_fill(ctx->neq, res_dev, 0.0, ctx->stream);
     for (const auto& g : ctx->groups)
         launch_transpose(g.shape, group_dev(ctx, g), wsigma_dev, res_dev, ctx->dOrig, ctx->stream);
@@ -2245,11 +2306,9 @@ namespace {
 // 1.44 M Q2 points 394 -> 167 us.
 void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStream_t s, bool split) {
     const int fmt = dep_format(ctx);
-    if (split && fmt == FMT_G64 && !ctx->update_mem) {
-        const PointState st = point_state(ctx);
-        for (int sh = 0; sh < SHAPE_COUNT; sh++)
-            launch_elem_dep(sh, split_dev(ctx, sh), u, st, ctx->dDep, ctx->npad, ctx->dEf, s);
-        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, ctx->dFlin, r, s);
+    if (split && fmt != FMT_D64 && !ctx->update_mem) {
+        elem_launches(ctx, EL_DEP, fmt, elem_args(ctx, u, ctx->dEf), s);
+        node_launch(ctx, ctx->dEf, ctx->dFlin, r, s);
         return;
     }
     if (fmt != FMT_D64) {
@@ -2265,8 +2324,7 @@ void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStre
         }
         return;
     }
-    for (const auto& g : ctx->groups)
-        launch_multiply(g.shape, group_dev(ctx, g), u, ctx->dStrain, ctx->dOrig, s);
+    strain_launches(ctx, u, ctx->dStrain, s);
     for (const auto& g : ctx->groups)
         launch_sigma(true, ctx->update_mem, g.shape, group_dev(ctx, g), ctx->npad, ctx->dStrain, ctx->dSigw, nullptr,
                      ctx->dOrig, point_state(ctx), s, ctx->dDep);
@@ -2365,7 +2423,7 @@ int ipf_residual_tangent(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if ((rc = ensure_solver_buffers(ctx))) return rc;
     residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream,
-                              ctx->have_geometry && ctx->npad <= kSplitPoints && split_stream(ctx));
+                              dep_format(ctx) != FMT_D64 && ctx->npad <= kSplitPoints && split_stream(ctx));
     ctx->have_tangent = true;
     ctx->dep32_ok = false;
     if ((rc = ensure_dep32(ctx))) return rc;
@@ -2559,9 +2617,9 @@ int ipf_tangent_apply(ipf_ctx* ctx, const double* v_dev, double* y_dev) {
     if (!v_dev || !y_dev) return fail(ctx, IPF_EINVAL, "ipf_tangent_apply: NULL pointer");
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if (format_geometric(ctx->tfmt) && ctx->npad <= kSplitPointsProduct && split_stream(ctx)) {
-        elem_tangent(ctx, v_dev, CgBeta{}, ctx->dEf, ctx->stream);
-        launch_nodes(ctx->neq, ctx->map_stride, ctx->dMap, ctx->dEf, nullptr, y_dev, ctx->stream);
+    if (split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPointsProduct && split_stream(ctx)) {
+        elem_launches(ctx, EL_TANGENT, ctx->tfmt, elem_args(ctx, v_dev, ctx->dEf), ctx->stream);
+        node_launch(ctx, ctx->dEf, nullptr, y_dev, ctx->stream);
     } else {
         tangent_product(ctx, v_dev, y_dev, ctx->stream);
     }

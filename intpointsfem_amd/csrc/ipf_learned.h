@@ -44,6 +44,31 @@ void launch_predict(const short* wbf, const float* par, const float* feat, int64
 
 }  // namespace mlp
 
+// Features (trial principal stresses over c, ln c, phi, psi, 1e3 alpha), exact
+// branch and 1e3 d_alpha of one point.  Only the eigenvalues of the trial
+// stress are wanted (spectral_ps's equal spectral's); the material's own
+// features come from the host.
+__device__ __forceinline__ void point_features(const double* e3, const double* ep, double alpha, const MatConst& m,
+                                               float* __restrict__ f, int& label, float& target) {
+    double s[6];
+    const double exx = e3[0] - ep[0], exy = e3[1] - ep[1], eyy = e3[2] - ep[2], ezz = 0 - ep[3];
+    s[XX] = m.lam2mu * exx + m.lambda * eyy + m.lambda * ezz;
+    s[YY] = m.lambda * exx + m.lam2mu * eyy + m.lambda * ezz;
+    s[ZZ] = m.lambda * exx + m.lambda * eyy + m.lam2mu * ezz;
+    s[XY] = m.mu * exy;
+    s[XZ] = s[YZ] = m.mu * 0.0;
+    double ev[3], vec[9], sp[3], hard = 0.0;
+    spectral_ps(s, ev, vec);
+    int mt, br;
+    project<false>(ev, sp, mt, br, hard, m, nullptr);
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4* out = reinterpret_cast<f4*>(f);
+    out[0] = f4{(float)(ev[0] / m.feat_c), (float)(ev[1] / m.feat_c), (float)(ev[2] / m.feat_c), m.feat_lnc};
+    out[1] = f4{m.feat_phi, m.feat_psi, (float)(alpha * 1e3), 0.f};
+    label = br;
+    target = (float)(hard * 1e3);
+}
+
 // Features [npts x FEAT_STRIDE], exact branch and 1e3 * d_alpha of every
 // point of one group at the trial state (nothing committed); reference
 // point order through orig.

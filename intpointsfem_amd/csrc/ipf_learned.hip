@@ -442,41 +442,8 @@ k_point_features(GroupDev g, int tp, const double* __restrict__ strain, const in
     if (o < 0) return;
     const MatConst& m = tile_material(g, tile);
     const double e3[3] = {strain[3 * o], strain[3 * o + 1], strain[3 * o + 2]};
-    double ep[4] = {st.ep0[P], st.ep1[P], st.ep2[P], st.ep3[P]};
-    const double alpha0 = st.alpha[P];
-    // trial stress and its principal values (point_sigma's first half)
-    double el[6];
-    el[XX] = e3[0] - ep[0];
-    el[XY] = e3[1] - ep[1];
-    el[XZ] = 0.0;
-    el[YY] = e3[2] - ep[2];
-    el[YZ] = 0.0;
-    el[ZZ] = 0 - ep[3];
-    double s[6];
-    s[XX] = m.lam2mu * el[XX] + m.lambda * el[YY] + m.lambda * el[ZZ];
-    s[YY] = m.lambda * el[XX] + m.lam2mu * el[YY] + m.lambda * el[ZZ];
-    s[ZZ] = m.lambda * el[XX] + m.lambda * el[YY] + m.lam2mu * el[ZZ];
-    s[XY] = m.mu * el[XY];
-    s[XZ] = m.mu * el[XZ];
-    s[YZ] = m.mu * el[YZ];
-    double ev[3], vec[9];
-    spectral(s, ev, vec);
-    double sp[3];
-    int mt, br;
-    double hard = 0.0;
-    project<false>(ev, sp, mt, br, hard, m, nullptr);
-    const double c = m.phi_c / (2. * m.cosphi);
-    float* f = feat + o * FEAT_STRIDE;
-    f[0] = (float)(ev[0] / c);
-    f[1] = (float)(ev[1] / c);
-    f[2] = (float)(ev[2] / c);
-    f[3] = (float)log(c);
-    f[4] = (float)asin(m.sinphi);
-    f[5] = (float)asin(m.sinpsi);
-    f[6] = (float)(alpha0 * 1e3);
-    f[7] = 0.f;
-    label[o] = br;
-    target[o] = (float)(hard * 1e3);
+    const double ep[4] = {st.ep0[P], st.ep1[P], st.ep2[P], st.ep3[P]};
+    point_features(e3, ep, st.alpha[P], m, feat + o * FEAT_STRIDE, label[o], target[o]);
 }
 
 }  // namespace

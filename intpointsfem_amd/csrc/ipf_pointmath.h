@@ -44,6 +44,8 @@ struct MatConst {
     double c_cot;           // c * (1/tan(phi))                    (FunctionsSigmaProjection.h:293,301)
     double apex_alpha;      // cos(phi)/sin(psi)                   (FunctionsSigmaProjection.h:300)
     double tan_plane[9], tan_right[9], tan_left[9];
+    double feat_c;                          // the cohesion as the predictor's features scale by it
+    float feat_lnc, feat_phi, feat_psi;     // ln c, phi, psi
 
     static MatConst make(double lambda, double mu, double mc_phi, double mc_psi, double c);
 };

@@ -4,6 +4,7 @@
 #include <cstdint>
 
 #include "ipf_kernels.h"
+#include "ipf_learned.h"
 
 namespace ipf {
 
@@ -16,34 +17,61 @@ constexpr int kSplitColors = 8;  // colors (and so groups of one shape) at most
 struct SplitDev {
     int nseg;
     int end[kSplitColors];
-    int tile0[kSplitColors];   // context tile (tmeta)
-    int pt0[kSplitColors];     // new point
-    int slot0[kSplitColors];   // element slot (corners)
-    int ent0[kSplitColors];    // node entry (node, ef)
+    int tile0[kSplitColors];      // context tile (tmeta)
+    int pt0[kSplitColors];        // new point
+    int slot0[kSplitColors];      // element slot (corners)
+    int ent0[kSplitColors];       // node entry (node, ef)
+    int64_t val0[kSplitColors];   // value of the compact FP64 B
     const int* tmeta;
     int64_t ntiles;
-    const double* geo;     // 8 corner values per element slot
+    const void* B;         // FMT_G64 / FMT_G32: 8 corner values per element slot; FMT_C64: the values
     const double* tab;     // shape table of the shape
     const int* node;       // x DoF per element slot and node
     const MatConst* mats;
 };
 
-// ef[entry] (two doubles) = the element's force on its node, fmt FMT_G64 / FMT_G32
-void launch_elem_residual(int fmt, int shape, bool fast, const SplitDev& g, const double* u, const PointState& st,
-                          double* ef, hipStream_t stream);
-// The residual's element forces and every point's w Dep (FMT_G64).
-void launch_elem_dep(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, int64_t npad,
-                     double* ef, hipStream_t stream);
-// With rz_old (a CG iteration, see ipf_kernels.h): v is z, and the vector
-// multiplied is z + beta p, formed as it is gathered.
+// What an element launch does (ipf_split.hip, k_elem).
+enum ElemOp {
+    EL_RESIDUAL = 0,   // u -> ef
+    EL_CERTIFIED = 1,  // the same, certified elastic points by their trial stress
+    EL_TANGENT = 2,    // u, dep -> ef of K u
+    EL_CG = 3,         // z, p, dep -> ef of K (z + beta p)
+    EL_DEP = 4,        // u -> ef, dep
+    EL_STRAIN = 5,     // u -> point (strains)
+    EL_FORCE = 6,      // point (w sigma) -> ef
+    EL_FEATURES = 7    // u -> feat, label, target
+};
+
+// z + beta p as a CG iteration gathers it (ipf_kernels.h).
 struct CgBeta {
     const double* p;
-    const double* rz_old;  // null: no CG, the product with v itself
+    const double* rz_old;
     const double* rz_partial;
     int nrz;
 };
-void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, double* dep,
-                         const float* dep32, int64_t npad, double* ef, hipStream_t stream);
+
+struct ElemArgs {
+    const double* u;
+    PointState st;
+    double* dep;          // w Dep, SoA, npad apart
+    const float* dep32;   // its FP32 copy (FMT_G32)
+    int64_t npad;
+    CgBeta cg;
+    double* ef;           // two doubles per node entry: the element's force on its node
+    double* point;        // 3 per point, reference order
+    const int64_t* orig;  // reference point of each new point
+    float* feat;
+    int* label;
+    float* target;
+};
+
+// fmt: FMT_G64 or FMT_C64; FMT_G32 for the residuals and the products.
+void launch_elem(int op, int fmt, int shape, const SplitDev& g, const ElemArgs& a, hipStream_t stream);
+
+// The return map of one shape's points: strains to w sigma and (wdep set)
+// w Dep, reference order.  Needs tile0, pt0, tmeta and mats of g only.
+void launch_stress(int shape, const SplitDev& g, const double* strain, double* wsigma, double* wdep,
+                   const int64_t* orig, const PointState& st, bool commit, hipStream_t stream);
 
 // map: stride (4 or 8) ints per node, one per color; filled with -1, then one
 // call per group (n0: the group's first node entry)

@@ -15,7 +15,25 @@ namespace ipf {
 
 namespace {
 
-enum ElemOp { EL_RESIDUAL = 0, EL_CERTIFIED = 1, EL_TANGENT = 2, EL_CG = 3, EL_DEP = 4 };
+// Values of the tile's points, N each, between LDS (point order) and the
+// reference order: an element's points are consecutive there, so the
+// wavefront reads and writes whole rows of it (lane by lane it would touch
+// every row N times).  oel: each element's first reference point.
+template <int N, int NIP>
+__device__ __forceinline__ void store_points(const double* sh, const int64_t* oel, int nv, double* __restrict__ dst) {
+    for (int t = threadIdx.x; t < nv * NIP * N; t += kWave) {
+        const int el = t / (NIP * N);
+        dst[N * oel[el] + (t - el * NIP * N)] = sh[t];
+    }
+}
+
+template <int N, int NIP>
+__device__ __forceinline__ void load_points(double* sh, const int64_t* oel, int nv, const double* __restrict__ src) {
+    for (int t = threadIdx.x; t < nv * NIP * N; t += kWave) {
+        const int el = t / (NIP * N);
+        sh[t] = src[N * oel[el] + (t - el * NIP * N)];
+    }
+}
 
 // One wavefront per tile: gather, strain, stress (or w Dep times the strain),
 // B^T products and the sums over each element's points, as k_residual_fmt /
@@ -27,21 +45,27 @@ enum ElemOp { EL_RESIDUAL = 0, EL_CERTIFIED = 1, EL_TANGENT = 2, EL_CG = 3, EL_D
 // the addresses read from a table: 20x20 Q2 7.8 us, so 6.3).
 template <int SHAPE, int FMT, int OP>
 __global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
-k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restrict__ dep,
-       const float* __restrict__ dep32, int64_t npad, CgBeta cg, dv2* __restrict__ ef) {
+k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
-    constexpr bool CG = OP == EL_CG, TAN = OP == EL_TANGENT || CG;
+    constexpr bool CG = OP == EL_CG, TAN = OP == EL_TANGENT || CG, FEAT = OP == EL_FEATURES;
+    constexpr bool STRESS = OP == EL_RESIDUAL || OP == EL_CERTIFIED || OP == EL_DEP;
+    constexpr bool GATHER = OP != EL_FORCE, FORCES = OP != EL_STRAIN && !FEAT;
+    constexpr bool POINTS = OP == EL_STRAIN || OP == EL_FORCE;  // per-point values in the reference order
+    const PointState& st = a.st;
     constexpr bool F32 = TAN && FMT == FMT_G32;
     constexpr int NSH = C::CE / 2;
     constexpr int H = 2 * ((NSH + 1) / 2), H2 = C::CE - H;
     constexpr int NE = C::ET * NSH;
     static_assert(NE <= kWave, "one node per lane");
-    __shared__ T lds[C::TP * H];
-    __shared__ double us[2 * NE];
+    __shared__ T lds[FORCES ? C::TP * H : 1];
+    __shared__ double us[GATHER ? 2 * NE : 1];
+    __shared__ double pts[POINTS ? 3 * C::TP : 1];
+    __shared__ int64_t oel[POINTS ? C::ET : 1];
     const int lane = threadIdx.x;
     const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
     int tile0 = g.tile0[0], pt0 = g.pt0[0], slot0 = g.slot0[0], ent0 = g.ent0[0];
+    int64_t val0 = g.val0[0];
 #pragma unroll
     for (int c = 1; c < kSplitColors; c++)
         if (c < g.nseg && t >= g.end[c - 1]) {
@@ -49,6 +73,7 @@ k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restri
             pt0 = g.pt0[c];
             slot0 = g.slot0[c];
             ent0 = g.ent0[c];
+            val0 = g.val0[c];
         }
     const int tm = g.tmeta[tile0 + t];
     const int64_t E0 = slot0 + t * C::ET, N0 = ent0 + t * NE;
@@ -58,53 +83,85 @@ k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restri
     const bool valid = slot && el < nv;
     // indexes, then the point's state, then the values the indexes address,
     // all outside branches (padding slots hold node DoF 0 and points of their own)
-    const int d = ld_stream(&g.node[N0 + min(lane, NE - 1)]) & kDofMask;
-    const WaveSum rz_sum(CG ? cg.nrz : 1, CG ? cg.rz_partial : u);
-    const double rz_old = CG ? *cg.rz_old : 0.0;
+    int d = 0;
+    if constexpr (GATHER) d = ld_stream(&g.node[N0 + min(lane, NE - 1)]) & kDofMask;
+    const WaveSum rz_sum(CG ? a.cg.nrz : 1, CG ? a.cg.rz_partial : u);
+    const double rz_old = CG ? *a.cg.rz_old : 0.0;
     const int64_t P = pt0 + t * C::TP + (slot ? lane : 0);
     double ep[4];
-    if constexpr (!TAN) {
+    if constexpr (STRESS || FEAT) {
         ep[0] = ld_stream(&st.ep0[P]);
         ep[1] = ld_stream(&st.ep1[P]);
         ep[2] = ld_stream(&st.ep2[P]);
         ep[3] = ld_stream(&st.ep3[P]);
     }
+    double alpha = 0.0;
+    if constexpr (FEAT) alpha = ld_stream(&st.alpha[P]);
+    int64_t o = -1;
+    if constexpr (POINTS || FEAT) o = ld_stream(&a.orig[P]);
     double dp[9];
     float dpf[9];
     if constexpr (TAN) {
 #pragma unroll
         for (int k = 0; k < 9; k++) {
             if constexpr (F32)
-                dpf[k] = ld_stream(&dep32[k * npad + P]);
+                dpf[k] = ld_stream(&a.dep32[k * a.npad + P]);
             else
-                dp[k] = ld_stream(&dep[k * npad + P]);
+                dp[k] = ld_stream(&a.dep[k * a.npad + P]);
         }
     }
-    double ux = u[d], uy = u[d + 1];
+    double ux = 0.0, uy = 0.0;
+    if constexpr (GATHER) {
+        ux = u[d];
+        uy = u[d + 1];
+    }
     if constexpr (CG) {
-        const double px = cg.p[d], py = cg.p[d + 1];
-        const double beta = cg_beta(rz_sum.get(cg.nrz, cg.rz_partial), rz_old);
+        const double px = a.cg.p[d], py = a.cg.p[d + 1];
+        const double beta = cg_beta(rz_sum.get(a.cg.nrz, a.cg.rz_partial), rz_old);
         ux = ux + beta * px;
         uy = uy + beta * py;
     }
     T b[C::NV];
     double w = 0.0;
-    if (valid) {
-        w = geom_values<SHAPE>(g.geo + 8 * E0, g.tab, 0, lane, b);
-    } else {
+    if constexpr (FmtTraits<FMT>::GEOM) {
+        if (valid) {
+            w = geom_values<SHAPE>(static_cast<const double*>(g.B) + 8 * E0, g.tab, 0, lane, b);
+        } else {
 #pragma unroll
-        for (int k = 0; k < C::NV; k++) b[k] = T(0);
+            for (int k = 0; k < C::NV; k++) b[k] = T(0);
+        }
+    } else {
+        if constexpr (STRESS) w = ld_stream(&st.w[P]);
+        if (slot) {
+            load_values<SHAPE, FMT>(static_cast<const T*>(g.B) + val0 + t * (int64_t)(C::NV * C::TP), 0, lane, b);
+        } else {
+#pragma unroll
+            for (int k = 0; k < C::NV; k++) b[k] = T(0);
+        }
     }
-    if (lane < NE) {
+    if (GATHER && lane < NE) {
         us[2 * lane] = ux;
         us[2 * lane + 1] = uy;
     }
+    if (POINTS && slot && lane == el * C::NIP) oel[el] = o;
     __syncthreads();
+    if constexpr (OP == EL_FORCE) {
+        load_points<3, C::NIP>(pts, oel, nv, a.point);
+        __syncthreads();
+    }
     double x[3] = {0.0, 0.0, 0.0};
     if (valid) {
         double e3[3];
-        strain_fmt<SHAPE, FMT>(b, us + el * C::CE, e3);
-        if constexpr (TAN) {
+        if constexpr (GATHER) strain_fmt<SHAPE, FMT>(b, us + el * C::CE, e3);
+        if constexpr (OP == EL_STRAIN) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) pts[3 * lane + k] = e3[k];
+        } else if constexpr (OP == EL_FORCE) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) x[k] = pts[3 * lane + k];
+        } else if constexpr (FEAT) {
+            point_features(e3, ep, alpha, g.mats[tm >> 8], a.feat + o * mlp::FEAT_STRIDE, a.label[o], a.target[o]);
+        } else if constexpr (TAN) {
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 if constexpr (F32) {
@@ -122,18 +179,22 @@ k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restri
         } else {
             const MatConst& mc = g.mats[tm >> 8];
             if constexpr (OP == EL_DEP) {
-                double alpha = 0.0, d9[9];
+                double d9[9];
                 int mt, br;
                 point_sigma<true>(e3, ep, alpha, mt, br, mc, w, x, d9);
 #pragma unroll
-                for (int k = 0; k < 9; k++) dep[k * npad + P] = d9[k];
+                for (int k = 0; k < 9; k++) a.dep[k * a.npad + P] = d9[k];
             } else if (!(OP == EL_CERTIFIED && certified_elastic(e3, ep, mc, w, x))) {
-                double alpha = 0.0;
                 int mt, br;
                 point_sigma<false>(e3, ep, alpha, mt, br, mc, w, x, nullptr);
             }
         }
     }
+    if constexpr (OP == EL_STRAIN) {
+        __syncthreads();
+        store_points<3, C::NIP>(pts, oel, nv, a.point);
+    }
+    if constexpr (!FORCES) return;
     // node rj of element re: its x and y columns, in the half that holds the node
     const int re = lane / NSH, rj = lane - re * NSH;
     const bool task = lane < NE && re < nv;
@@ -164,7 +225,76 @@ k_elem(SplitDev g, const double* __restrict__ u, PointState st, double* __restri
         }
         f = dv2{double(fx), double(fy)};
     }
-    if (task) ef[N0 + lane] = f;
+    if (task) reinterpret_cast<dv2*>(a.ef)[N0 + lane] = f;
+}
+
+// The separate steps and the features, per 716 k Q2 points (dense B, a launch
+// per color, every point's three values stored lane by lane -> now): strain
+// 4 x 16.9 -> 17.9 us, force 4 x 19.0 + clear 4.8 -> 18.5 + nodes 7.4, stress
+// 4 x 10.9 -> 31.4 (bound by the return map's instructions); features of 1.44 M
+// points 4 x (33.0 + 16.7) -> 49.9.
+
+// The return map of a shape's points, strains and stresses (DEP: w Dep too) in
+// the reference order through LDS rows (store_points).
+template <int SHAPE, bool DEP>
+__global__ void __launch_bounds__(kWave, DEP ? 3 : 4)
+k_stress(SplitDev g, const double* __restrict__ strain, double* __restrict__ wsigma, double* __restrict__ wdep,
+         const int64_t* __restrict__ orig, PointState st, int commit) {
+    constexpr int NIP = shape_nip(SHAPE), ET = shape_et(SHAPE), TP = shape_tp(SHAPE), N = DEP ? 9 : 3;
+    __shared__ double sh[N * TP];
+    __shared__ int64_t oel[ET];
+    const int lane = threadIdx.x;
+    const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
+    int tile0 = g.tile0[0], pt0 = g.pt0[0];
+#pragma unroll
+    for (int c = 1; c < kSplitColors; c++)
+        if (c < g.nseg && t >= g.end[c - 1]) {
+            tile0 = g.tile0[c];
+            pt0 = g.pt0[c];
+        }
+    const int tm = g.tmeta[tile0 + t];
+    const int nv = tm & 255, el = lane / NIP;
+    const bool slot = lane < TP, valid = slot && el < nv;
+    const int64_t P = pt0 + t * TP + (slot ? lane : 0);
+    const int64_t o = ld_stream(&orig[P]);
+    double ep[4] = {ld_stream(&st.ep0[P]), ld_stream(&st.ep1[P]), ld_stream(&st.ep2[P]), ld_stream(&st.ep3[P])};
+    double alpha = commit ? st.alpha[P] : 0.0;
+    const double w = ld_stream(&st.w[P]);
+    if (slot && lane == el * NIP) oel[el] = o;
+    __syncthreads();
+    load_points<3, NIP>(sh, oel, nv, strain);
+    __syncthreads();
+    double ws[3] = {0.0, 0.0, 0.0}, d9[9];
+    if (valid) {
+        const double e3[3] = {sh[3 * lane], sh[3 * lane + 1], sh[3 * lane + 2]};
+        int mt, br;
+        point_sigma<DEP>(e3, ep, alpha, mt, br, g.mats[tm >> 8], w, ws, d9);
+        if (commit) {
+            st.ep0[P] = ep[0];
+            st.ep1[P] = ep[1];
+            st.ep2[P] = ep[2];
+            st.ep3[P] = ep[3];
+            st.alpha[P] = alpha;
+            st.mtype[P] = (signed char)mt;
+            st.branch[P] = (signed char)br;
+        }
+    }
+    __syncthreads();
+    if (valid) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) sh[3 * lane + k] = ws[k];
+    }
+    __syncthreads();
+    store_points<3, NIP>(sh, oel, nv, wsigma);
+    if constexpr (DEP) {
+        __syncthreads();
+        if (valid) {
+#pragma unroll
+            for (int k = 0; k < 9; k++) sh[9 * lane + k] = d9[k];
+        }
+        __syncthreads();
+        store_points<9, NIP>(sh, oel, nv, wdep);
+    }
 }
 
 // map[node * 4 NQ + color] = the entry of ef that the color's element adds to
@@ -282,53 +412,57 @@ k_nodes_cg(int64_t n, const int* __restrict__ map, const dv2* __restrict__ ef, c
 }
 
 template <int FMT, int OP>
-void elem(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, const float* dep32,
-          int64_t npad, const CgBeta& cg, double* ef, hipStream_t s) {
+void elem(int shape, const SplitDev& g, const ElemArgs& a, hipStream_t s) {
     dispatch_shape(shape, [&](auto sc) {
         constexpr int S = decltype(sc)::value;
-        hipLaunchKernelGGL((k_elem<S, FMT, OP>), dim3((unsigned)g.ntiles), dim3(kWave), 0, s, g, u, st, dep, dep32,
-                           npad, cg, reinterpret_cast<dv2*>(ef));
+        hipLaunchKernelGGL((k_elem<S, FMT, OP>), dim3((unsigned)g.ntiles), dim3(kWave), 0, s, g, a.u, a);
     });
+}
+
+template <int FMT>
+void elem_op(int op, int shape, const SplitDev& g, const ElemArgs& a, hipStream_t s) {
+    switch (op) {
+        case EL_RESIDUAL: elem<FMT, EL_RESIDUAL>(shape, g, a, s); break;
+        case EL_CERTIFIED: elem<FMT, EL_CERTIFIED>(shape, g, a, s); break;
+        case EL_TANGENT: elem<FMT, EL_TANGENT>(shape, g, a, s); break;
+        case EL_CG: elem<FMT, EL_CG>(shape, g, a, s); break;
+        default: break;
+    }
+    if constexpr (FMT != FMT_G32) {
+        switch (op) {
+            case EL_DEP: elem<FMT, EL_DEP>(shape, g, a, s); break;
+            case EL_STRAIN: elem<FMT, EL_STRAIN>(shape, g, a, s); break;
+            case EL_FORCE: elem<FMT, EL_FORCE>(shape, g, a, s); break;
+            case EL_FEATURES: elem<FMT, EL_FEATURES>(shape, g, a, s); break;
+            default: break;
+        }
+    }
 }
 
 }  // namespace
 
-void launch_elem_residual(int fmt, int shape, bool fast, const SplitDev& g, const double* u, const PointState& st,
-                          double* ef, hipStream_t s) {
+void launch_elem(int op, int fmt, int shape, const SplitDev& g, const ElemArgs& a, hipStream_t s) {
     if (g.ntiles == 0) return;
-    if (fmt == FMT_G64) {
-        if (fast)
-            elem<FMT_G64, EL_CERTIFIED>(shape, g, u, st, nullptr, nullptr, 0, CgBeta{}, ef, s);
-        else
-            elem<FMT_G64, EL_RESIDUAL>(shape, g, u, st, nullptr, nullptr, 0, CgBeta{}, ef, s);
-    } else if (fmt == FMT_G32) {
-        if (fast)
-            elem<FMT_G32, EL_CERTIFIED>(shape, g, u, st, nullptr, nullptr, 0, CgBeta{}, ef, s);
-        else
-            elem<FMT_G32, EL_RESIDUAL>(shape, g, u, st, nullptr, nullptr, 0, CgBeta{}, ef, s);
-    }
+    if (fmt == FMT_G64)
+        elem_op<FMT_G64>(op, shape, g, a, s);
+    else if (fmt == FMT_C64)
+        elem_op<FMT_C64>(op, shape, g, a, s);
+    else if (fmt == FMT_G32)
+        elem_op<FMT_G32>(op, shape, g, a, s);
 }
 
-void launch_elem_dep(int shape, const SplitDev& g, const double* u, const PointState& st, double* dep, int64_t npad,
-                     double* ef, hipStream_t s) {
-    if (g.ntiles) elem<FMT_G64, EL_DEP>(shape, g, u, st, dep, nullptr, npad, CgBeta{}, ef, s);
-}
-
-void launch_elem_tangent(int fmt, int shape, const SplitDev& g, const double* v, const CgBeta& cg, double* dep,
-                         const float* dep32, int64_t npad, double* ef, hipStream_t s) {
+void launch_stress(int shape, const SplitDev& g, const double* strain, double* wsigma, double* wdep,
+                   const int64_t* orig, const PointState& st, bool commit, hipStream_t s) {
     if (g.ntiles == 0) return;
-    const PointState none{};
-    if (fmt == FMT_G64) {
-        if (cg.rz_old)
-            elem<FMT_G64, EL_CG>(shape, g, v, none, dep, dep32, npad, cg, ef, s);
+    const dim3 grid((unsigned)g.ntiles), block(kWave);
+    dispatch_shape(shape, [&](auto sc) {
+        constexpr int S = decltype(sc)::value;
+        if (wdep)
+            hipLaunchKernelGGL((k_stress<S, true>), grid, block, 0, s, g, strain, wsigma, wdep, orig, st, commit ? 1 : 0);
         else
-            elem<FMT_G64, EL_TANGENT>(shape, g, v, none, dep, dep32, npad, cg, ef, s);
-    } else if (fmt == FMT_G32) {
-        if (cg.rz_old)
-            elem<FMT_G32, EL_CG>(shape, g, v, none, dep, dep32, npad, cg, ef, s);
-        else
-            elem<FMT_G32, EL_TANGENT>(shape, g, v, none, dep, dep32, npad, cg, ef, s);
-    }
+            hipLaunchKernelGGL((k_stress<S, false>), grid, block, 0, s, g, strain, wsigma, wdep, orig, st,
+                               commit ? 1 : 0);
+    });
 }
 
 void launch_fill_int(int64_t n, int* p, int v, hipStream_t s) {

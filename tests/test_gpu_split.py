@@ -122,3 +122,58 @@ def test_cg_solution(gpu, mesh):
     ctx.synchronize()
     res = np.where(mask, 0.0, b - y.cpu().numpy())
     assert np.linalg.norm(res) <= 10 * rtol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("mesh", [(1, 1, 1, 1.0), (7, 9, 1, 1.2), (1, 1, 2, 1.0), (5, 6, 2, 1.2), (4, 3, 3, 1.3)],
+                         ids=str)
+def test_stored_blocks_and_corners_agree(gpu, mesh):
+    """Every element launch from the stored compact values and from the
+    corners (bit-identical values, so bit-identical results), and the strains
+    and forces against numpy's dense blocks (1e-14 of the terms' sum per
+    column, a few columns)."""
+    import torch
+    m = wb.make_mesh(mesh)
+    sm = ipf.StructMatrix(m, device=0)
+    b, ix, s, d = sm.export_blocks(), sm.export_indexes(), sm.sizes(), m.material()
+    stored = ipf.DeviceContext(device=0)
+    stored.transfer_data(b["row_sizes"], b["col_sizes"], b["matrix_position"], b["row_first"], b["col_first"],
+                         b["storage"], ix["dof_indexes"], ix["color_indexes"], s["ncolor"], s["neq"], ix["weight"])
+    stored.set_material(d["lambda"], d["mu"], d["phi"], d["psi"], d["cohesion"])
+    stored.set_rhs_linear(ix["rhs_linear"])
+    u = wb.lame_displacement(m.nodes(), wb.normal_stress(10), scale=4.0)
+    du = torch.as_tensor(u, dtype=torch.float64, device=gpu)
+    n, neq = s["npts"], s["neq"]
+
+    def zeros(k, t=torch.float64):
+        return torch.full((k,), 7, dtype=t, device=gpu)
+    out = []
+    for ctx in (sm.context(), stored):
+        r, rt, y, f = (zeros(neq) for _ in range(4))
+        e, w, wd, w2 = zeros(3 * n), zeros(3 * n), zeros(9 * n), zeros(3 * n)
+        feat, br, tg = zeros(8 * n, torch.float32), zeros(n, torch.int32), zeros(n, torch.float32)
+        torch.cuda.synchronize()
+        ctx.residual(du, r)
+        ctx.residual_tangent(du, rt)
+        ctx.tangent_apply(du, y)
+        ctx.multiply(du, e)
+        ctx.compute_sigma(e, w)
+        ctx.compute_sigma_dep(e, w2, wd)
+        ctx.multiply_transpose(w, f)
+        ctx.point_features(du, feat, br, tg)
+        ctx.synchronize()
+        out.append([t.cpu().numpy() for t in (r, rt, y, e, w, w2, wd, f, feat, br, tg)])
+    for x, z in zip(*out):
+        assert np.isfinite(x).all() and np.array_equal(x, z)
+    r, rt, y, e, w, w2, wd, f, *_ = out[0]
+    assert np.array_equal(r, rt) and np.array_equal(w, w2)
+    nb, C = s["nblocks"], int(b["col_sizes"][0])
+    B = b["storage"].reshape(nb, -1, C)
+    dof = np.asarray(ix["dof_indexes"]).reshape(nb, C)
+    bound = 1e-14 * C
+    ref, size = (B * u[dof][:, None, :]).sum(-1), (np.abs(B) * np.abs(u[dof])[:, None, :]).sum(-1)
+    assert (np.abs(e.reshape(ref.shape) - ref) <= bound * size).all()
+    t = B * w.reshape(nb, -1)[:, :, None]
+    ref, size = np.zeros(neq), np.zeros(neq)
+    np.add.at(ref, dof, -t.sum(1))
+    np.add.at(size, dof, np.abs(t).sum(1))
+    assert (np.abs(f - ref) <= 1e-14 * B.shape[1] * size).all()
