@@ -158,8 +158,8 @@ int ipf_info(const ipf_ctx *ctx, int64_t out[8]);
  * (TPZElastoPlasticIntPointsStructMatrix.cpp:137-154) ->
  * TPZNumericalIntegrator::ResidualIntegration (TPZNumericalIntegrator.cpp:107-128).
  * One fused kernel per element color: gather, B.u, return map, B^T (w sigma)
- * and the color's atomic-free accumulation into r -- or, up to 2 million
- * points of geometric B with aligned (x, y) DoF pairs in at most 8 colors, one
+ * and the color's atomic-free accumulation into r -- or, up to 400,000
+ * points of geometric or compact FP64 B with aligned (x, y) DoF pairs in at most 8 colors, one
  * element launch per shape and one node launch that sums in color order (the
  * same bits; calls that overlap on several streams, and calls under capture,
  * keep the launch per color).  r is overwritten entirely (its previous contents are never read); u and r must not

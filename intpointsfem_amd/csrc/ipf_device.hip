@@ -469,20 +469,21 @@ void release_data(ipf_ctx* ctx) {
     ctx->bytes = 0;
 }
 
-// Up to how many points a residual or a CG iteration (and a single product)
-// takes the element / node launches.  Below, a color's launch leaves most of
-// the chip idle and the launches' own times add up; above, the element forces
-// no longer stay in the Infinity Cache and their write and read cost what the
-// colored launches' repeated r costs.  us per residual, colored -> element /
-// node: Q2 14 k points 23.2 -> 9.7, 90 k 25.3 -> 12.3, 810 k 58.6 -> 45.6,
-// 1.44 M 82.7 -> 73.8, 2.7 M 129.7 -> 127.9, 5.8 M 253 -> 264; Q1 2.56 M
-// 106 -> 100; Q3 2.56 M 159 -> 154.  Per CG iteration (nine launches -> three):
-// Q2 14 k 23.8 -> 12.9, 90 k 29.1 -> 16.8, 1.44 M 100.6 -> 85.1, 2.7 M 152 ->
-// 144, 5.8 M 280 -> 315.  Per product: 90 k 17.1 -> 9.0, 810 k 35.3 -> 32.1,
-// 2.7 M 87.9 -> 90.1.  Per residual with tangent: Q2 90 k 42.3 -> 19.5,
-// 1.44 M 149 -> 142, 2.7 M 239 -> 243; Q1 2.56 M 197 -> 207.  Products right after a residual and tangent (cold caches) 1.44 M
-// points already lose 2 us.
-constexpr int64_t kSplitPoints = 2000000, kSplitPointsProduct = 1000000;
+// Up to how many points a residual, a residual with tangent or a product
+// (kSplitPoints), and a CG iteration (kSplitPointsCg), take the element / node
+// launches.  Below, a color's launch leaves most of the chip idle and the
+// launches' own times add up; above, the element forces no longer stay in the
+// Infinity Cache and their write and read cost what the colored launches'
+// repeated r costs.  us per residual, colored -> element / node, one context
+// alone: Q2 14 k points 23.2 -> 9.7, 90 k 25.3 -> 12.3, 360 k 34.8 -> 27.3,
+// 810 k 58.6 -> 45.6, 1.44 M 82.7 -> 73.8, 5.8 M 253 -> 264.  Where several
+// contexts keep the chip busy (three on three streams) the gain ends earlier:
+// Q2 90 k 12.6 -> 6.6, 360 k 18.4 -> 17.1, 810 k 34.3 -> 37.2, Q1 360 k 16.2 ->
+// 15.6, 640 k 23.4 -> 25.2, Q3 314 k 22.6 -> 18.4, 640 k 32.9 -> 35.0; products
+// the same.  A CG iteration (nine launches -> three) waits for itself either
+// way: Q2 14 k 23.8 -> 12.9, 90 k 29.1 -> 16.8, 1.44 M 100.6 -> 85.1, 2.7 M
+// 152 -> 144, 5.8 M 280 -> 315.
+constexpr int64_t kSplitPoints = 400000, kSplitPointsCg = 2000000;
 
 // The B formats of the element launches: geometric or compact FP64.
 bool split_format(const ipf_ctx* ctx, int fmt) {
@@ -491,7 +492,7 @@ bool split_format(const ipf_ctx* ctx, int fmt) {
 
 // Whether the CG takes the element / node launches (three per iteration).
 bool cg_split(const ipf_ctx* ctx) {
-    return ctx->split_ok && ctx->npad <= kSplitPoints && split_format(ctx, ctx->tfmt);
+    return ctx->split_ok && ctx->npad <= kSplitPointsCg && split_format(ctx, ctx->tfmt);
 }
 
 constexpr int kScal = 16;  // CG / Newton scalars in dScal
@@ -2617,7 +2618,7 @@ int ipf_tangent_apply(ipf_ctx* ctx, const double* v_dev, double* y_dev) {
     if (!v_dev || !y_dev) return fail(ctx, IPF_EINVAL, "ipf_tangent_apply: NULL pointer");
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if (split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPointsProduct && split_stream(ctx)) {
+    if (split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
         elem_launches(ctx, EL_TANGENT, ctx->tfmt, elem_args(ctx, v_dev, ctx->dEf), ctx->stream);
         node_launch(ctx, ctx->dEf, nullptr, y_dev, ctx->stream);
     } else {
