@@ -48,7 +48,7 @@ IPF_HD QuadMap quad_map(const double* X, double xi, double eta) {
     }
     QuadMap m;
     m.det = xx * ye - xe * yx;
-    const double inv = 1.0 / m.det;
+    const double inv = quot(1.0, recip(m.det));  // 1 / det
     m.a = ye * inv;
     m.b = -(yx * inv);
     m.c = -(xe * inv);

@@ -52,75 +52,6 @@ struct MatConst {
 
 // ---------------------------------------------------------------- spectral
 
-// FunctionsSpectralDecomp.h:7-20
-IPF_HD double normalize6(double* s) {
-    double maxel = s[0];
-#pragma unroll
-    for (int i = 1; i < 6; i++)
-        if (fabs(s[i]) > fabs(maxel)) maxel = s[i];
-    if (maxel != 0) {
-#pragma unroll
-        for (int i = 0; i < 6; i++) s[i] /= maxel;
-    }
-    return maxel;
-}
-
-// FunctionsSpectralDecomp.h:25-56 (row 3 uses sxy + syz as the reference does)
-IPF_HD void gershgorin(const double* s, double& upper_out, double& lower_out) {
-    const double row_1 = s[XY] + s[XZ];
-    const double lo0 = s[XX] - fabs(row_1), up0 = s[XX] + fabs(row_1);
-    const double row_2 = s[XY] + s[YZ];
-    const double lo1 = s[YY] - fabs(row_2), up1 = s[YY] + fabs(row_2);
-    const double row_3 = s[XY] + s[YZ];
-    const double lo2 = s[ZZ] - fabs(row_3), up2 = s[ZZ] + fabs(row_3);
-    double up = up0, lo = lo0;
-    if (up1 > up) up = up1;
-    if (lo1 < lo) lo = lo1;
-    if (up2 > up) up = up2;
-    if (lo2 < lo) lo = lo2;
-    upper_out = up;
-    lower_out = lo;
-}
-
-// Cubic of FunctionsSpectralDecomp.h:75-77, evaluated left to right.
-IPF_HD double cubic(double x, const double* s, double sxy2, double sxz2, double syz2) {
-    return -x * x * x - sxz2 * s[YY] - sxy2 * s[ZZ] - syz2 * s[XX] + 2 * s[XY] * s[XZ] * s[YZ] +
-           s[XX] * s[YY] * s[ZZ] + x * x * (s[XX] + s[YY] + s[ZZ]) +
-           x * (sxy2 + sxz2 + syz2 - s[XX] * s[YY] - s[XX] * s[ZZ] - s[YY] * s[ZZ]);
-}
-
-// FunctionsSpectralDecomp.h:61-111: Newton from each Gershgorin bound
-// (20 iterations, |f| > 1e-11), third root from the trace, descending sort.
-IPF_HD void eigenvalues_newton(double up, double lo, const double* s, double maxel, double* ev) {
-    const double sxy2 = s[XY] * s[XY];
-    const double sxz2 = s[XZ] * s[XZ];
-    const double syz2 = s[YZ] * s[YZ];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        double x = (i == 0) ? up : lo;
-        double f = cubic(x, s, sxy2, sxz2, syz2);
-        double res = fabs(f);
-        int it = 0;
-        while (it < 20 && res > 10e-12) {
-            const double df = -3 * x * x + sxy2 + sxz2 + syz2 - s[XX] * s[YY] - s[XX] * s[ZZ] - s[YY] * s[ZZ] +
-                              2 * x * (s[XX] + s[YY] + s[ZZ]);
-            x -= f / df;
-            f = cubic(x, s, sxy2, sxz2, syz2);
-            res = fabs(f);
-            it++;
-        }
-        ev[i] = x;
-    }
-    ev[2] = s[XX] + s[YY] + s[ZZ] - ev[0] - ev[1];
-    ev[0] *= maxel;
-    ev[1] *= maxel;
-    ev[2] *= maxel;
-    // i = 0: j = 1, 2; i = 1: j = 2 (FunctionsSpectralDecomp.h:102-110)
-    if (ev[0] < ev[1]) { const double a = ev[0]; ev[0] = ev[1]; ev[1] = a; }
-    if (ev[0] < ev[2]) { const double a = ev[0]; ev[0] = ev[2]; ev[2] = a; }
-    if (ev[1] < ev[2]) { const double a = ev[1]; ev[1] = ev[2]; ev[2] = a; }
-}
-
 // FunctionsSpectralDecomp.h:116-150
 // The eigenvector helpers return their vectors as values (V3) and the callers
 // store all nine components once, unconditionally: with results written
@@ -179,43 +110,6 @@ IPF_HD void eigvec_double(const double* s, double lam, V3& vec1, V3& vec2) {
     vec2 = V3{b0 / n2, b1 / n2, b2 / n2};
 }
 
-// FunctionsSpectralDecomp.h:217-256 followed by the normalise/scale-back of
-// :261-268.  s is normalised on entry and scaled back by maxel here.
-IPF_HD void eigenvectors6(double* s, const double* ev, double* vec, double maxel) {
-#pragma unroll
-    for (int i = 0; i < 6; i++) s[i] *= maxel;
-    V3 a{1., 0., 0.}, b{0., 1., 0.}, c{0., 0., 1.};  // three equal eigenvalues: the identity
-    if (!((ev[0] == ev[1]) && (ev[1] == ev[2]))) {
-        if (ev[0] != ev[1] && ev[0] != ev[2]) {
-            a = eigvec_simple(s, ev[0]);
-        } else if (ev[0] == ev[1]) {
-            eigvec_double(s, ev[0], a, b);
-        } else if (ev[0] == ev[2]) {
-            eigvec_double(s, ev[0], a, c);
-        }
-        if (ev[1] != ev[0] && ev[1] != ev[2]) {
-            b = eigvec_simple(s, ev[1]);
-        } else if (ev[1] == ev[2]) {
-            eigvec_double(s, ev[1], b, c);
-        }
-        if (ev[2] != ev[0] && ev[2] != ev[1]) {
-            c = eigvec_simple(s, ev[2]);
-        }
-    }
-    vec[0] = a.x; vec[1] = a.y; vec[2] = a.z;
-    vec[3] = b.x; vec[4] = b.y; vec[5] = b.z;
-    vec[6] = c.x; vec[7] = c.y; vec[8] = c.z;
-}
-
-// FunctionsSpectralDecomp.h:261-268 (s is modified in place like the reference)
-IPF_HD void spectral(double* s, double* ev, double* vec) {
-    const double maxel = normalize6(s);
-    double up, lo;
-    gershgorin(s, up, lo);
-    eigenvalues_newton(up, lo, s, maxel, ev);
-    eigenvectors6(s, ev, vec, maxel);
-}
-
 // ---------------------------------------------------------------- plane strain
 //
 // spectral_ps: spectral() for a tensor whose XZ and YZ components are +0 (the
@@ -236,30 +130,78 @@ IPF_HD void spectral(double* s, double* ev, double* vec) {
 //     the (finite, >= 1) norm leaves unchanged.
 // Non-finite or degenerate cases (a zero minor, NaN) take the general code.
 
-IPF_HD double cubic_ps(double x, const double* s, double sxy2) {
-    return -x * x * x - sxy2 * s[ZZ] + s[XX] * s[YY] * s[ZZ] + x * x * (s[XX] + s[YY] + s[ZZ]) +
-           x * (sxy2 - s[XX] * s[YY] - s[XX] * s[ZZ] - s[YY] * s[ZZ]);
+// Quotients by one divisor and square roots, correctly rounded like the
+// operators (and so the same bits), without the operators' scaling of extreme
+// operands: a reciprocal with error e^3 from the hardware's (e <= 5e-8), the
+// quotient corrected by its exact remainder.  7 instructions instead of 11 and
+// the waits between them, 3 for every further quotient by the same divisor; 10
+// instead of 18 for a root.  For divisors, quotients and radicands between
+// 2^-1000 and 2^1000 (zero numerators included); stresses between 1e-150 and
+// 1e150 stay inside (their minors, products of two, are within 1e-300 and
+// 1e300 or exactly 0, which the callers keep out).
+struct Recip {
+    double d, r;
+};
+
+IPF_HD Recip recip(double d) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double r0 = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, r0, 1.0);
+    return Recip{d, __builtin_fma(r0, __builtin_fma(e, e, e), r0)};
+#else
+    return Recip{d, 0.0};
+#endif
 }
 
+IPF_HD double quot(double n, const Recip& R) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double q = n * R.r;
+    return __builtin_fma(__builtin_fma(-R.d, q, n), R.r, q);
+#else
+    return n / R.d;
+#endif
+}
+
+IPF_HD double sqrt_in_range(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+    double s = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, s, 0.5);
+    h = __builtin_fma(h, e, h);
+    s = __builtin_fma(s, e, s);
+    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+    return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+#else
+    return sqrt(x);
+#endif
+}
+
+// The reference's Newton steps on the cubic with its loop constants named, each
+// expression summed in the reference's order (2 x T = x (2 T): a power of 2).
+// The quotient f / f' is taken by recip: outside the spectrum, where the
+// iterates stay, |f| > 1e-11 implies |f'| >= |f|^(2/3) > 4e-8, and all values
+// are of order 1.
 IPF_HD void eigenvalues_newton_ps(double up, double lo, const double* s, double maxel, double* ev) {
     const double sxy2 = s[XY] * s[XY];
+    const double p = s[XX] * s[YY], q = s[XX] * s[ZZ], r = s[YY] * s[ZZ];
+    const double T = s[XX] + s[YY] + s[ZZ], T2 = 2 * T;
+    const double A = sxy2 * s[ZZ], B = p * s[ZZ], C = sxy2 - p - q - r;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         double x = (i == 0) ? up : lo;
-        double f = cubic_ps(x, s, sxy2);
-        double res = fabs(f);
+        double x2 = x * x;
+        double f = -(x2 * x) - A + B + x2 * T + x * C;
         int it = 0;
-        while (it < 20 && res > 10e-12) {
-            const double df = -3 * x * x + sxy2 - s[XX] * s[YY] - s[XX] * s[ZZ] - s[YY] * s[ZZ] +
-                              2 * x * (s[XX] + s[YY] + s[ZZ]);
-            x -= f / df;
-            f = cubic_ps(x, s, sxy2);
-            res = fabs(f);
+        while (it < 20 && fabs(f) > 10e-12) {
+            const double df = -3 * x * x + sxy2 - p - q - r + x * T2;
+            x -= quot(f, recip(df));
+            x2 = x * x;
+            f = -(x2 * x) - A + B + x2 * T + x * C;
             it++;
         }
         ev[i] = x;
     }
-    ev[2] = s[XX] + s[YY] + s[ZZ] - ev[0] - ev[1];
+    ev[2] = T - ev[0] - ev[1];
     ev[0] *= maxel;
     ev[1] *= maxel;
     ev[2] *= maxel;
@@ -268,36 +210,25 @@ IPF_HD void eigenvalues_newton_ps(double up, double lo, const double* s, double 
     if (ev[1] < ev[2]) { const double a = ev[1]; ev[1] = ev[2]; ev[2] = a; }
 }
 
+// eigvec_simple with sxz = syz = +-0: the xy minor's vector is (0, 0, 1), and
+// in the other two branches the z component is a zero.  A vanishing or
+// non-finite largest minor takes the general code.
 IPF_HD V3 eigvec_simple_ps(const double* s, double lam) {
-    const double d0 = (s[XX] - lam) * (s[YY] - lam) - s[XY] * s[XY];
-    const double d1 = (s[XX] - lam) * (s[ZZ] - lam) - s[XZ] * s[XZ];
-    const double d2 = (s[YY] - lam) * (s[ZZ] - lam) - s[YZ] * s[YZ];
+    const double ax = s[XX] - lam, ay = s[YY] - lam, az = s[ZZ] - lam;
+    const double d0 = ax * ay - s[XY] * s[XY];
+    const double d1 = ax * az;
+    const double d2 = ay * az;
     double maxdet = fabs(d0);
-    if (fabs(d1) > fabs(maxdet)) maxdet = fabs(d1);
-    if (fabs(d2) > fabs(maxdet)) maxdet = fabs(d2);
-    double v0, v1, v2;
-    if (maxdet == fabs(d0)) {
-        const double t0 = -(s[YY] - lam) * s[XZ] + s[XY] * s[YZ];
-        const double t1 = -(s[XX] - lam) * s[YZ] + s[XY] * s[XZ];
-        if ((d0 > 0.0 || d0 < 0.0) && t0 == 0.0 && t1 == 0.0) {
-            // (1/d0) t: a zero with sign(d0) * sign(t); norm sqrt(0 + 0 + 1) = 1
-            return V3{d0 > 0.0 ? t0 : -t0, d0 > 0.0 ? t1 : -t1, 1.0};
-        }
-        v0 = 1 / d0 * t0;
-        v1 = 1 / d0 * t1;
-        v2 = 1;
-    } else if (maxdet == fabs(d1)) {
-        v0 = 1 / d1 * (-(s[ZZ] - lam) * s[XY] + s[XZ] * s[YZ]);
-        v1 = 1;
-        v2 = 1 / d1 * (-(s[XX] - lam) * s[YZ] + s[XY] * s[XZ]);
-    } else {
-        v0 = 1;
-        v1 = 1 / d2 * (-(s[ZZ] - lam) * s[XY] + s[XZ] * s[YZ]);
-        v2 = 1 / d2 * (-(s[YY] - lam) * s[XZ] + s[XY] * s[YZ]);
-    }
-    const double norm = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
-    // v2 / norm for a zero v2 and a finite norm (>= 1 here) is v2 itself
-    return V3{v0 / norm, v1 / norm, (v2 == 0.0 && norm >= 1.0 && norm <= 1.7976931348623157e308) ? v2 : v2 / norm};
+    if (fabs(d1) > maxdet) maxdet = fabs(d1);
+    if (fabs(d2) > maxdet) maxdet = fabs(d2);
+    if (!__builtin_isnormal(maxdet)) return eigvec_simple(s, lam);
+    if (maxdet == fabs(d0)) return V3{0.0, 0.0, 1.0};
+    const bool first = maxdet == fabs(d1);  // (v, 1, 0), else (1, v, 0)
+    const double v = quot(1.0, recip(first ? d1 : d2)) * (-az * s[XY]);
+    const double v2 = v * v;
+    const Recip norm = recip(sqrt_in_range(v2 + 1.0));
+    const double a = quot(v, norm), b = quot(1.0, norm);
+    return first ? V3{a, b, 0.0} : V3{b, a, 0.0};
 }
 
 IPF_HD void eigenvectors6_ps(double* s, const double* ev, double* vec, double maxel) {
@@ -334,10 +265,11 @@ IPF_HD void spectral_ps(double* s, double* ev, double* vec) {
     if (fabs(s[YY]) > fabs(maxel)) maxel = s[YY];
     if (fabs(s[ZZ]) > fabs(maxel)) maxel = s[ZZ];
     if (maxel != 0) {
-        s[XX] /= maxel;
-        s[XY] /= maxel;
-        s[YY] /= maxel;
-        s[ZZ] /= maxel;
+        const Recip m = recip(maxel);
+        s[XX] = quot(s[XX], m);
+        s[XY] = quot(s[XY], m);
+        s[YY] = quot(s[YY], m);
+        s[ZZ] = quot(s[ZZ], m);
         const double z = maxel > 0 ? 0.0 : (maxel < 0 ? -0.0 : s[XZ] / maxel);
         s[XZ] = z;
         s[YZ] = z;
