@@ -250,13 +250,13 @@ struct ipf_ctx {
     bool split_ok = false;
     int map_stride = 0;
     SplitDev split[SHAPE_COUNT];
+    double* dEf = nullptr;      // the element forces, then the map (one allocation)
     int* dMap = nullptr;
-    double* dEf = nullptr;
     double* dEfS = nullptr;
     int64_t nent = 0;           // node entries of all element slots
     bool ef_bound = false;
     hipStream_t ef_stream = nullptr;
-    double* dU = nullptr;       // staging for host-pointer calls
+    double* dU = nullptr;       // staging for host-pointer calls: u, then r (dR)
     double* dR = nullptr;
     int64_t bytes = 0;
 
@@ -394,8 +394,8 @@ void release_patch(ipf_ctx* ctx) {
 }
 
 void release_split(ipf_ctx* ctx) {
-    dev_free(ctx->dMap);
     dev_free(ctx->dEf);
+    ctx->dMap = nullptr;
     for (auto& d : ctx->split) d = SplitDev{};
     ctx->split_ok = false;
     ctx->ef_bound = false;
@@ -423,7 +423,7 @@ void release_data(ipf_ctx* ctx) {
     release_split(ctx);
     dev_free(ctx->dEfS);
     dev_free(ctx->dU);
-    dev_free(ctx->dR);
+    ctx->dR = nullptr;
     dev_free(ctx->dDep);
     dev_free(ctx->dDep32);
     ctx->dep32_ok = false;
@@ -780,12 +780,13 @@ void build_split(ipf_ctx* ctx) {
     }
     const int64_t nnode = (ctx->neq + 1) / 2;
     const std::string err = ctx->err;
-    if (dev_alloc(ctx, &ctx->dMap, nnode * stride) || dev_alloc(ctx, &ctx->dEf, 2 * nent)) {
+    if (dev_alloc(ctx, &ctx->dEf, 2 * nent + (nnode * stride + 1) / 2)) {
         (void)hipGetLastError();
         ctx->err = err;
         release_split(ctx);
         return;
     }
+    ctx->dMap = reinterpret_cast<int*>(ctx->dEf + 2 * nent);
     launch_fill_int(nnode * stride, ctx->dMap, -1, ctx->stream);
     for (const auto& g : ctx->groups) {
         GroupDev d = group_dev(ctx, g);
@@ -1445,13 +1446,14 @@ static int transfer_impl(ipf_ctx* ctx, int64_t nblocks, const int* row_sizes, co
         (rc = dev_alloc(ctx, &ctx->dEp[3], npad)) || (rc = dev_alloc(ctx, &ctx->dAlpha, npad)) ||
         (rc = dev_alloc(ctx, &ctx->dMtype, npad)) || (rc = dev_alloc(ctx, &ctx->dBranch, npad)) ||
         (rc = dev_alloc(ctx, &ctx->dOrig, npad)) || (rc = dev_alloc(ctx, &ctx->dFlin, neq)) ||
-        (rc = dev_alloc(ctx, &ctx->dU, neq)) || (rc = dev_alloc(ctx, &ctx->dR, neq)) ||
+        (rc = dev_alloc(ctx, &ctx->dU, 2 * neq)) ||
         (rc = dev_alloc(ctx, &ctx->dTmeta, ntile_all)) || (rc = dev_alloc(ctx, &ctx->dNewOf, npts)) ||
         (rc = dev_alloc(ctx, &ctx->dPmat, npad)) ||
         (fold && (rc = dev_alloc(ctx, &ctx->dDofR, nd))) || (pairs && (rc = dev_alloc(ctx, &ctx->dNodeR, nd / 2)))) {
         release_data(ctx);
         return rc;
     }
+    ctx->dR = ctx->dU + neq;
     int64_t ntab = 0;
     if (geo) {
         for (int sh = 0; sh < SHAPE_COUNT; sh++) {

@@ -125,9 +125,11 @@ __device__ __forceinline__ void strain_fmt(const typename FC<SHAPE, FMT>::T* b, 
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
     if constexpr (FmtTraits<FMT>::COMPACT) {
-        T a0 = T(0), a1 = T(0), a2 = T(0);
+        // (the dense sums start from 0: a zero's sign apart, from the first term)
+        T a0 = b[0] * T(ue[0]), a1 = b[1] * T(ue[0]), a2 = b[1] * T(ue[1]);
+        a1 = a1 + b[0] * T(ue[1]);
 #pragma unroll
-        for (int a = 0; a < C::CE / 2; a++) {
+        for (int a = 1; a < C::CE / 2; a++) {
             const T dx = b[2 * a], dy = b[2 * a + 1];
             const T ux = T(ue[2 * a]), uy = T(ue[2 * a + 1]);
             a0 = a0 + dx * ux;
@@ -147,6 +149,19 @@ __device__ __forceinline__ void strain_fmt(const typename FC<SHAPE, FMT>::T* b, 
             e3[k] = double(acc);
         }
     }
+}
+
+// Row stride of the staged partials: every lane writes its row of W values of
+// B bytes in 16-byte pieces, eight lanes at a time, and reads pairs down the
+// columns.  A stride of W put the rows of Q3 (16 FP64 values) on one bank in
+// four (960 of 1,296 LDS cycles per wavefront were conflicts, and the LDS bound
+// the launch); W rounded up to an odd multiple of 16 bytes spreads eight rows
+// over all 64 banks.
+constexpr int row_stride(int w, int bytes) {
+    const int per = 16 / bytes;
+    if (w % 2) return w;  // single values
+    int q = (w + per - 1) / per;
+    return (q % 2 ? q : q + 1) * per;
 }
 
 // Columns [J0, J1) of one point's B^T (w sigma) partials into row[j - J0].
@@ -183,7 +198,7 @@ __device__ __forceinline__ void bt_cols(const typename FC<SHAPE, FMT>::T* b, con
 }
 
 // One lane's column sum: the partials L of element e's points in column jj of
-// the staged half (W columns), summed in point order and added negated to
+// the staged half (rows W values apart), summed in point order and added negated to
 // r[d] (TPZNumericalIntegrator::MultiplyTranspose's y = -B^T x); rv = r[d],
 // read by the caller ahead of time.  Each lane owns one column sum per half
 // (ET * W <= 64 for every shape), and the color's elements share no DoF, so

@@ -38,9 +38,10 @@ struct QuadMap {
 IPF_HD QuadMap quad_map(const double* X, double xi, double eta) {
     const double dxi[4] = {-(1 - eta) / 4, (1 - eta) / 4, (1 + eta) / 4, -(1 + eta) / 4};
     const double deta[4] = {-(1 - xi) / 4, -(1 + xi) / 4, (1 + xi) / 4, (1 - xi) / 4};
-    double xx = 0, xe = 0, yx = 0, ye = 0;  // dx/dxi, dx/deta, dy/dxi, dy/deta
+    // dx/dxi, dx/deta, dy/dxi, dy/deta
+    double xx = dxi[0] * X[0], xe = deta[0] * X[0], yx = dxi[0] * X[1], ye = deta[0] * X[1];
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
+    for (int c = 1; c < 4; c++) {
         xx += dxi[c] * X[2 * c];
         xe += deta[c] * X[2 * c];
         yx += dxi[c] * X[2 * c + 1];

@@ -47,7 +47,7 @@ namespace {
 // npad apart): one launch per color in place of strain, stress and force
 // launches over the stored dense B.
 template <int SHAPE, int FMT, bool COMMIT, bool PAIR, bool FAST, bool DEP = false>
-__global__ void __launch_bounds__(kWave, (DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
+__global__ void __launch_bounds__(kWave, (DEP ? (FC<SHAPE, FMT>::CE <= 8 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
 k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict__ u, double* __restrict__ r,
                const double* __restrict__ flin, PointState st, double* __restrict__ dep, int64_t npad) {
     static_assert(!(FAST && (COMMIT || DEP)), "the certified elastic path commits nothing and has no tangent");
@@ -58,12 +58,16 @@ k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict
     // holds the first ceil(NSH / 2) nodes), else CE / 2 columns each
     constexpr int H = PAIR ? 2 * ((NSH + 1) / 2) : C::CE / 2;
     constexpr int H2 = C::CE - H;
+    constexpr int RS = row_stride(H, sizeof(T)), RS2 = row_stride(H2, sizeof(T));
     static_assert(C::ET * NSH <= kWave, "one column sum (PAIR: node) per lane and half");
     constexpr bool R_EARLY = (SHAPE == SHAPE_Q3 || (SHAPE == SHAPE_Q2 && FAST)) && !COMMIT;
     constexpr int NE = PAIR ? C::ET * NSH : C::ET * C::CE;  // index entries per tile
-    __shared__ T lds[C::TP * H];
+    __shared__ T lds[C::TP * (RS > RS2 ? RS : RS2)];
     __shared__ double us[C::ET * C::CE];
-    __shared__ int dsx[NE];
+    // PAIR: lane re NSH + rj holds its own node's index (DEP and FAST at Q2, short of registers:
+    // through LDS like the others)
+    constexpr bool OWN = PAIR && !DEP && !(FAST && SHAPE == SHAPE_Q2);
+    __shared__ int dsx[OWN ? 1 : NE];
     const int lane = threadIdx.x;
     const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
     const int el = lane / C::NIP;
@@ -118,7 +122,7 @@ k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict
     for (int k = 0; k < NG; k++) {
         const int t = lane + k * kWave;
         if ((k == 0 && !PAIR) || t < NE) {
-            dsx[t] = dl[k];
+            if (!OWN) dsx[t] = dl[k];
             if (PAIR) {
                 us[2 * t] = ul[k];
                 us[2 * t + 1] = vl[k];
@@ -138,7 +142,7 @@ k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict
     auto start = [&](int de, int off) -> double { return (de < 0 ? flin : r)[(de & kDofMask) + off]; };
     auto request_r = [&](double& r0, double& r1) {
         if (PAIR) {
-            const int de = dsx[re * NSH + rj];
+            const int de = OWN ? dl[0] : dsx[lane];
             r0 = start(de, 0);
             r1 = start(de, 1);
         } else {
@@ -175,28 +179,28 @@ k_residual_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict
     }
     // otherwise both r values now, in flight during the first half's products
     if (!R_EARLY && task) request_r(r0, r1);
-    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, ws, lds + lane * H);
+    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, ws, lds + lane * RS);
     __syncthreads();
     if (PAIR) {
         if (task && first_half) {
-            const int d = dsx[re * NSH + rj] & kDofMask;
-            reduce_lane<SHAPE, FMT, H>(lds, re, 2 * rj, d, r0, r);
-            reduce_lane<SHAPE, FMT, H>(lds, re, 2 * rj + 1, d + 1, r1, r);
+            const int d = (OWN ? dl[0] : dsx[lane]) & kDofMask;
+            reduce_lane<SHAPE, FMT, RS>(lds, re, 2 * rj, d, r0, r);
+            reduce_lane<SHAPE, FMT, RS>(lds, re, 2 * rj + 1, d + 1, r1, r);
         }
     } else if (task) {
-        reduce_lane<SHAPE, FMT, H>(lds, re, rj, dsx[re * C::CE + rj] & kDofMask, r0, r);
+        reduce_lane<SHAPE, FMT, RS>(lds, re, rj, dsx[re * C::CE + rj] & kDofMask, r0, r);
     }
     __syncthreads();
-    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, ws, lds + lane * H2);
+    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, ws, lds + lane * RS2);
     __syncthreads();
     if (PAIR) {
         if (task && !first_half) {
-            const int d = dsx[re * NSH + rj] & kDofMask;
-            reduce_lane<SHAPE, FMT, H2>(lds, re, 2 * rj - H, d, r0, r);
-            reduce_lane<SHAPE, FMT, H2>(lds, re, 2 * rj - H + 1, d + 1, r1, r);
+            const int d = (OWN ? dl[0] : dsx[lane]) & kDofMask;
+            reduce_lane<SHAPE, FMT, RS2>(lds, re, 2 * rj - H, d, r0, r);
+            reduce_lane<SHAPE, FMT, RS2>(lds, re, 2 * rj - H + 1, d + 1, r1, r);
         }
     } else if (task) {
-        reduce_lane<SHAPE, FMT, H2>(lds, re, rj, dsx[re * C::CE + H + rj] & kDofMask, r1, r);
+        reduce_lane<SHAPE, FMT, RS2>(lds, re, rj, dsx[re * C::CE + H + rj] & kDofMask, r1, r);
     }
 }
 
@@ -216,11 +220,12 @@ k_tangent_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict_
     // staged halves of the columns as in k_residual_fmt
     constexpr int H = PAIR ? 2 * ((NSH + 1) / 2) : C::CE / 2;
     constexpr int H2 = C::CE - H;
+    constexpr int RS = row_stride(H, sizeof(T)), RS2 = row_stride(H2, sizeof(T));
     static_assert(C::ET * NSH <= kWave, "one column sum (PAIR: node) per lane and half");
     constexpr int NE = PAIR ? C::ET * NSH : C::ET * C::CE;
-    __shared__ T lds[C::TP * H];
+    __shared__ T lds[C::TP * (RS > RS2 ? RS : RS2)];
     __shared__ double vs[C::ET * C::CE];
-    __shared__ int dsx[NE];
+    __shared__ int dsx[PAIR ? 1 : NE];  // PAIR: lane re NSH + rj holds its own node's index
     const int lane = threadIdx.x;
     const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
     const int el = lane / C::NIP;
@@ -262,7 +267,7 @@ k_tangent_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict_
     for (int k = 0; k < NG; k++) {
         const int t = lane + k * kWave;
         if ((k == 0 && !PAIR) || t < NE) {
-            dsx[t] = dl[k];
+            if (!PAIR) dsx[t] = dl[k];
             if (PAIR) {
                 vs[2 * t] = vl[k];
                 vs[2 * t + 1] = vl2[k];
@@ -298,7 +303,7 @@ k_tangent_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict_
         }
         if (task) {
             if (PAIR) {
-                const int de = dsx[re * NSH + rj];
+                const int de = dl[0];
                 y0 = start(de, 0);
                 y1 = start(de, 1);
             } else {
@@ -328,28 +333,28 @@ k_tangent_fmt(GroupDev g, const void* __restrict__ Bv, const double* __restrict_
             }
         }
     }
-    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, x, lds + lane * H);
+    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, x, lds + lane * RS);
     __syncthreads();
     if (PAIR) {
         if (task && first_half) {
-            const int d = dsx[re * NSH + rj] & kDofMask;
-            reduce_lane<SHAPE, FMT, H>(lds, re, 2 * rj, d, y0, y);
-            reduce_lane<SHAPE, FMT, H>(lds, re, 2 * rj + 1, d + 1, y1, y);
+            const int d = dl[0] & kDofMask;
+            reduce_lane<SHAPE, FMT, RS>(lds, re, 2 * rj, d, y0, y);
+            reduce_lane<SHAPE, FMT, RS>(lds, re, 2 * rj + 1, d + 1, y1, y);
         }
     } else if (task) {
-        reduce_lane<SHAPE, FMT, H>(lds, re, rj, dsx[re * C::CE + rj] & kDofMask, y0, y);
+        reduce_lane<SHAPE, FMT, RS>(lds, re, rj, dsx[re * C::CE + rj] & kDofMask, y0, y);
     }
     __syncthreads();
-    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, x, lds + lane * H2);
+    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, x, lds + lane * RS2);
     __syncthreads();
     if (PAIR) {
         if (task && !first_half) {
-            const int d = dsx[re * NSH + rj] & kDofMask;
-            reduce_lane<SHAPE, FMT, H2>(lds, re, 2 * rj - H, d, y0, y);
-            reduce_lane<SHAPE, FMT, H2>(lds, re, 2 * rj - H + 1, d + 1, y1, y);
+            const int d = dl[0] & kDofMask;
+            reduce_lane<SHAPE, FMT, RS2>(lds, re, 2 * rj - H, d, y0, y);
+            reduce_lane<SHAPE, FMT, RS2>(lds, re, 2 * rj - H + 1, d + 1, y1, y);
         }
     } else if (task) {
-        reduce_lane<SHAPE, FMT, H2>(lds, re, rj, dsx[re * C::CE + H + rj] & kDofMask, y1, y);
+        reduce_lane<SHAPE, FMT, RS2>(lds, re, rj, dsx[re * C::CE + H + rj] & kDofMask, y1, y);
     }
 }
 
@@ -442,13 +447,13 @@ k_residual_patch(PatchDev p, const double* __restrict__ u, double* __restrict__ 
     using C = FC<SHAPE, FMT_G64>;
     constexpr int ET = C::ET, NIP = C::NIP, CE = C::CE, TP = C::TP;
     constexpr int NSH = CE / 2, PE = NW * ET, MAXN = patch_max_nodes(SHAPE, NW), NT = NW * kWave;
-    constexpr int H = CE / 2, H2 = CE - H;
+    constexpr int H = CE / 2, H2 = CE - H, RS = row_stride(H, 8), RS2 = row_stride(H2, 8), RSM = RS > RS2 ? RS : RS2;
     constexpr int MAXC = 4;  // contributions requested up front; more are read at the end
     static_assert(ET * H <= kWave && ET * H2 <= kWave, "one column sum per lane and half");
     static_assert(MAXN <= NT, "one patch node per thread");
     __shared__ double us[2 * MAXN];
     __shared__ double es[PE * CE];
-    __shared__ double stg[NW * TP * H];
+    __shared__ double stg[NW * TP * RSM];
     __shared__ unsigned short lns[PE * NSH];
     const int tid = threadIdx.x, w = tid / kWave, lane = tid - w * kWave;
     // XCD-contiguous patch ranges for the exact return map (800x800 Q2:
@@ -513,24 +518,24 @@ k_residual_patch(PatchDev p, const double* __restrict__ u, double* __restrict__ 
         }
     }
     // element column sums, half the columns at a time through the wave's own staging
-    double* L = stg + w * TP * H;
+    double* L = stg + w * TP * RSM;
     const int re = lane / H, rj = lane - re * H;
-    if (slot) bt_cols<SHAPE, FMT_G64, 0, H>(b, ws, L + lane * H);
+    if (slot) bt_cols<SHAPE, FMT_G64, 0, H>(b, ws, L + lane * RS);
     wave_lds_sync();
     if (lane < ET * H && re < nv) {
-        double f = L[(re * NIP) * H + rj];
+        double f = L[(re * NIP) * RS + rj];
 #pragma unroll
-        for (int ip = 1; ip < NIP; ip++) f = f + L[(re * NIP + ip) * H + rj];
+        for (int ip = 1; ip < NIP; ip++) f = f + L[(re * NIP + ip) * RS + rj];
         es[(w * ET + re) * CE + rj] = f;
     }
     wave_lds_sync();
     const int re2 = lane / H2, rj2 = lane - re2 * H2;
-    if (slot) bt_cols<SHAPE, FMT_G64, H, CE>(b, ws, L + lane * H2);
+    if (slot) bt_cols<SHAPE, FMT_G64, H, CE>(b, ws, L + lane * RS2);
     wave_lds_sync();
     if (lane < ET * H2 && re2 < nv) {
-        double f = L[(re2 * NIP) * H2 + rj2];
+        double f = L[(re2 * NIP) * RS2 + rj2];
 #pragma unroll
-        for (int ip = 1; ip < NIP; ip++) f = f + L[(re2 * NIP + ip) * H2 + rj2];
+        for (int ip = 1; ip < NIP; ip++) f = f + L[(re2 * NIP + ip) * RS2 + rj2];
         es[(w * ET + re2) * CE + H + rj2] = f;
     }
     __syncthreads();

@@ -44,7 +44,7 @@ __device__ __forceinline__ void load_points(double* sh, const int64_t* oel, int 
 // and last round trip (a product with w Dep requested after the gather and
 // the addresses read from a table: 20x20 Q2 7.8 us, so 6.3).
 template <int SHAPE, int FMT, int OP>
-__global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
+__global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 8 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
 k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
@@ -56,9 +56,10 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     constexpr bool F32 = TAN && FMT == FMT_G32;
     constexpr int NSH = C::CE / 2;
     constexpr int H = 2 * ((NSH + 1) / 2), H2 = C::CE - H;
+    constexpr int RS = row_stride(H, sizeof(T)), RS2 = row_stride(H2, sizeof(T));
     constexpr int NE = C::ET * NSH;
     static_assert(NE <= kWave, "one node per lane");
-    __shared__ T lds[FORCES ? C::TP * H : 1];
+    __shared__ T lds[FORCES ? C::TP * (RS > RS2 ? RS : RS2) : 1];
     __shared__ double us[GATHER ? 2 * NE : 1];
     __shared__ double pts[POINTS ? 3 * C::TP : 1];
     __shared__ int64_t oel[POINTS ? C::ET : 1];
@@ -200,28 +201,28 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     const bool task = lane < NE && re < nv;
     const bool first = rj < H / 2;
     dv2 f = {0.0, 0.0};
-    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, x, lds + lane * H);
+    if (slot) bt_cols<SHAPE, FMT, 0, H>(b, x, lds + lane * RS);
     __syncthreads();
     if (task && first) {
-        const T* L = lds + re * C::NIP * H + 2 * rj;
+        const T* L = lds + re * C::NIP * RS + 2 * rj;
         T fx = L[0], fy = L[1];
 #pragma unroll
         for (int ip = 1; ip < C::NIP; ip++) {
-            fx = fx + L[ip * H];
-            fy = fy + L[ip * H + 1];
+            fx = fx + L[ip * RS];
+            fy = fy + L[ip * RS + 1];
         }
         f = dv2{double(fx), double(fy)};
     }
     __syncthreads();
-    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, x, lds + lane * H2);
+    if (slot) bt_cols<SHAPE, FMT, H, C::CE>(b, x, lds + lane * RS2);
     __syncthreads();
     if (task && !first) {
-        const T* L = lds + re * C::NIP * H2 + 2 * rj - H;
+        const T* L = lds + re * C::NIP * RS2 + 2 * rj - H;
         T fx = L[0], fy = L[1];
 #pragma unroll
         for (int ip = 1; ip < C::NIP; ip++) {
-            fx = fx + L[ip * H2];
-            fy = fy + L[ip * H2 + 1];
+            fx = fx + L[ip * RS2];
+            fy = fy + L[ip * RS2 + 1];
         }
         f = dv2{double(fx), double(fy)};
     }
