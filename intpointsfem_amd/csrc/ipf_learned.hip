@@ -487,97 +487,138 @@ namespace ipf {
 namespace {
 
 constexpr int kSortBlock = IPF_SORT_BLOCK;
+constexpr int kSortRound = 4 * kSortBlock;  // keys per round of the scatter
 
-// counting sort of keys in [0, NK): per-block histograms
-template <int NK>
-__global__ void __launch_bounds__(kSortBlock) k_key_hist(const int* __restrict__ key, int64_t n, int* __restrict__ hist) {
-    __shared__ int h[NK];
-    if (threadIdx.x < NK) h[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * kSortBlock + threadIdx.x;
-    if (i < n) {
-        const int k = key[i];
-        atomicAdd(&h[(k >= 0 && k < NK) ? k : NK - 1], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x < NK) hist[(int64_t)blockIdx.x * NK + threadIdx.x] = h[threadIdx.x];
-}
+__device__ __forceinline__ int clamp_key(int k, int nk) { return (k >= 0 && k < nk) ? k : nk - 1; }
 
-// exclusive offsets: key-major, then block order.  One block of 1024
-// threads; thread t owns a contiguous chunk of the block histograms.
-constexpr int kScanThreads = 1024;
+// Counting sort of keys in [0, NK): block b counts the keys of its chunk, then
+// every block of the scatter sums the counts before it itself (NK columns of
+// at most kSortMaxBlocks rows out of L2) -- no scan between the two launches.
+// hist[k * nb + b].
 template <int NK>
-__global__ void __launch_bounds__(kScanThreads) k_key_scan(int* __restrict__ hist, int nblocks) {
-    __shared__ long long part[kScanThreads][NK];
-    __shared__ long long base[NK];
-    const int t = threadIdx.x;
-    const int chunk = (nblocks + kScanThreads - 1) / kScanThreads;
-    const int b0 = min(nblocks, t * chunk), b1 = min(nblocks, b0 + chunk);
-    long long sum[NK];
+__global__ void __launch_bounds__(kSortBlock)
+k_key_hist(const int* __restrict__ key, int64_t n, int64_t chunk, int* __restrict__ hist) {
+    constexpr int NW = kSortBlock / kWave;
+    __shared__ int part[NW][NK];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+    int c[NK];
 #pragma unroll
-    for (int k = 0; k < NK; k++) sum[k] = 0;
-    for (int b = b0; b < b1; b++)
+    for (int k = 0; k < NK; k++) c[k] = 0;
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kSortBlock) {
+        const int v = clamp_key(key[i], NK);
 #pragma unroll
-        for (int k = 0; k < NK; k++) sum[k] += hist[(int64_t)b * NK + k];
-#pragma unroll
-    for (int k = 0; k < NK; k++) part[t][k] = sum[k];
-    __syncthreads();
-    if (t < NK) {  // per key: exclusive prefix over the chunks, then the key totals
-        long long run = 0;
-        for (int i = 0; i < kScanThreads; i++) {
-            const long long c = part[i][t];
-            part[i][t] = run;
-            run += c;
-        }
-        base[t] = run;
+        for (int k = 0; k < NK; k++) c[k] += v == k;
     }
-    __syncthreads();
-    if (t == 0) {
-        long long acc = 0;
-        for (int k = 0; k < NK; k++) {
-            const long long c = base[k];
-            base[k] = acc;
-            acc += c;
-        }
-    }
-    __syncthreads();
 #pragma unroll
     for (int k = 0; k < NK; k++) {
-        long long run = base[k] + part[t][k];
-        for (int b = b0; b < b1; b++) {
-            const int c = hist[(int64_t)b * NK + k];
-            hist[(int64_t)b * NK + k] = (int)run;
-            run += c;
-        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) c[k] += __shfl_xor(c[k], o, kWave);
+        if (lane == 0) part[wave][k] = c[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < NK) {
+        int s = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) s += part[w][threadIdx.x];
+        hist[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
     }
 }
 
-// stable scatter: rank of an element among the same keys before it in its
-// block, from wavefront ballots and per-wave counts
+// Stable scatter of the block's chunk, kSortRound keys at a time, four in a row
+// per thread: the counts of the keys before a thread's are one 64-bit scan of
+// packed 12-bit fields (at most 256 keys per wavefront).
 template <int NK>
-__global__ void __launch_bounds__(kSortBlock) k_key_scatter(const int* __restrict__ key, int64_t n,
-                                                           const int* __restrict__ offs, int* __restrict__ order) {
+__global__ void __launch_bounds__(kSortBlock)
+k_key_scatter(const int* __restrict__ key, int64_t n, int64_t chunk, const int* __restrict__ hist,
+              int* __restrict__ order) {
+    static_assert(NK <= 5, "12-bit fields of one 64-bit word");
     constexpr int NW = kSortBlock / kWave;
-    __shared__ int wc[NW][NK];
+    __shared__ unsigned long long wc[2][NW];
+    __shared__ int before_part[NW][NK], total_part[NW][NK];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int64_t i = (int64_t)blockIdx.x * kSortBlock + threadIdx.x;
-    int k = -1;
-    if (i < n) {
-        k = key[i];
-        if (k < 0 || k >= NK) k = NK - 1;
-    }
-    int rank_in_wave = 0;
+    const int nb = gridDim.x, me = blockIdx.x;
+    const int64_t i0 = (int64_t)me * chunk, i1 = min(n, i0 + chunk);
+    int k[4];
+    auto request = [&](int64_t i) {  // branch-free: keys past the chunk are read as its last and not used
+#pragma unroll
+        for (int q = 0; q < 4; q++) k[q] = key[min(i + q, i1 - 1)];
+    };
+    request(i0 + 4 * (int)threadIdx.x);
+    int bs[NK], ts[NK];
+#pragma unroll
+    for (int j = 0; j < NK; j++) bs[j] = ts[j] = 0;
+    for (int b = threadIdx.x; b < nb; b += kSortBlock)
+#pragma unroll
+        for (int j = 0; j < NK; j++) {
+            const int h = hist[(int64_t)j * nb + b];
+            ts[j] += h;
+            bs[j] += b < me ? h : 0;
+        }
 #pragma unroll
     for (int j = 0; j < NK; j++) {
-        const unsigned long long b = __ballot(k == j);
-        if (lane == 0) wc[wave][j] = __popcll(b);
-        if (k == j) rank_in_wave = __popcll(b & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            ts[j] += __shfl_xor(ts[j], o, kWave);
+            bs[j] += __shfl_xor(bs[j], o, kWave);
+        }
+        if (lane == 0) {
+            before_part[wave][j] = bs[j];
+            total_part[wave][j] = ts[j];
+        }
     }
     __syncthreads();
-    if (i < n) {
-        int before = 0;
-        for (int w = 0; w < wave; w++) before += wc[w][k];
-        order[offs[(int64_t)blockIdx.x * NK + k] + before + rank_in_wave] = (int)i;
+    int before[NK];  // where key j's next element goes
+    int base = 0;
+#pragma unroll
+    for (int j = 0; j < NK; j++) {
+        int b = 0, t = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            b += before_part[w][j];
+            t += total_part[w][j];
+        }
+        before[j] = base + b;
+        base += t;
+    }
+    int buf = 0;
+    for (int64_t r0 = i0; r0 < i1; r0 += kSortRound, buf ^= 1) {
+        const int64_t i = r0 + 4 * (int)threadIdx.x;
+        int v[4];
+        unsigned long long mine = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            v[q] = i + q < i1 ? clamp_key(k[q], NK) : NK;
+            if (v[q] < NK) mine += 1ull << (12 * v[q]);
+        }
+        if (r0 + kSortRound < i1) request(i + kSortRound);
+        unsigned long long incl = mine;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const unsigned long long up = __shfl_up(incl, o, kWave);
+            if (lane >= o) incl += up;
+        }
+        if (lane == kWave - 1) wc[buf][wave] = incl;
+        __syncthreads();  // one barrier per round: the next one writes the other buffer
+        const unsigned long long excl = incl - mine;
+        int pos[NK];
+#pragma unroll
+        for (int j = 0; j < NK; j++) {
+            int round = 0, ahead = 0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const int c = (int)((wc[buf][w] >> (12 * j)) & 0xfff);
+                ahead += w < wave ? c : 0;
+                round += c;
+            }
+            pos[j] = before[j] + ahead + (int)((excl >> (12 * j)) & 0xfff);
+            before[j] += round;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int j = 0; j < NK; j++)
+                if (v[q] == j) order[pos[j]++] = (int)(i + q);
     }
 }
 
@@ -614,14 +655,24 @@ k_sigma_order(int64_t n, const int* __restrict__ order, const int64_t* __restric
 
 }  // namespace
 
+// Chunks of whole rounds, at most kSortMaxBlocks of them: enough blocks to fill
+// the chip, few enough rows that every block can sum them.  1.44 M keys:
+// histograms 8.5 + scan by one block 46 + scatter 6.1 us -> 5.9 + 10.3.
+constexpr int kSortMaxBlocks = 1024;
+
+static int64_t sort_chunk(int64_t n) {
+    const int64_t rounds = (n + kSortRound - 1) / kSortRound;
+    return (rounds + kSortMaxBlocks - 1) / kSortMaxBlocks * kSortRound;
+}
+
 int key_sort_blocks(int64_t n) { return (int)((n + kSortBlock - 1) / kSortBlock); }
 
 void launch_branch_order(const int* key, int64_t n, int* hist, int* order, hipStream_t s) {
     if (n == 0) return;
-    const int nb = key_sort_blocks(n);
-    hipLaunchKernelGGL(k_key_hist<IPF_NBRANCH>, dim3(nb), dim3(kSortBlock), 0, s, key, n, hist);
-    hipLaunchKernelGGL(k_key_scan<IPF_NBRANCH>, dim3(1), dim3(kScanThreads), 0, s, hist, nb);
-    hipLaunchKernelGGL(k_key_scatter<IPF_NBRANCH>, dim3(nb), dim3(kSortBlock), 0, s, key, n, hist, order);
+    const int64_t chunk = sort_chunk(n);
+    const int nb = (int)((n + chunk - 1) / chunk);
+    hipLaunchKernelGGL(k_key_hist<IPF_NBRANCH>, dim3(nb), dim3(kSortBlock), 0, s, key, n, chunk, hist);
+    hipLaunchKernelGGL(k_key_scatter<IPF_NBRANCH>, dim3(nb), dim3(kSortBlock), 0, s, key, n, chunk, hist, order);
 }
 
 void launch_sigma_order(int64_t n, const int* order, const int64_t* new_of, const int* pmat, const MatConst* mats,
