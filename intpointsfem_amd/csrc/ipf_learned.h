@@ -30,13 +30,14 @@ constexpr int OFF_B3 = OFF_W3 + H * OUTP;
 constexpr int NPAR = OFF_B3 + OUTP;
 constexpr int NPAR_TRAINABLE = IN * H + H + H * H + H + H * OUT + OUT;  // 5062
 
-// gradient of the mean loss over n samples into per-wavefront slots
-// (nblocks * 4 slots of NPAR floats) and summed losses (nblocks * 4 doubles)
+// gradient of the mean loss over n samples into per-block slots (nblocks slots
+// of NPAR floats) and summed losses (nblocks doubles)
 void launch_grad(const short* wbf, const float* par, const float* feat, const int* label, const float* target,
                  int64_t n, int nblocks, float* slots, double* loss_slots, hipStream_t s);
-// grad = sum of the slots in order; with adam, one Adam step on par / m1 / m2
+// grad = sum of the slots in a fixed order, the summed loss (a double) behind
+// its NPAR floats; with adam, one Adam step on par / m1 / m2
 // (bias corrections bc1 = 1 - b1^t, bc2 = 1 - b2^t) and BF16 copies in wbf
-void launch_reduce(const float* slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
+void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
                    bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s);
 void launch_refresh(const float* par, short* wbf, hipStream_t s);
 void launch_predict(const short* wbf, const float* par, const float* feat, int64_t n, int nblocks, int* branch,

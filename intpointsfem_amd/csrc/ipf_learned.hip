@@ -84,16 +84,22 @@ struct WaveLDS {
 };
 
 struct WeightsLDS {
-    short W1[INP][H];
-    short W2[H][H];
-    short W3[H][OUTP];
+    alignas(16) short W1[INP][H];
+    alignas(16) short W2[H][H];
+    alignas(16) short W3[H][OUTP];
     float b1[H], b2[H], b3[OUTP];
 };
 
+// 16 bytes at a time: the matrices start on multiples of 8 values in wbf.
 __device__ void load_weights(WeightsLDS& w, const short* __restrict__ wbf, const float* __restrict__ par) {
-    for (int i = threadIdx.x; i < INP * H; i += blockDim.x) (&w.W1[0][0])[i] = wbf[OFF_W1 + i];
-    for (int i = threadIdx.x; i < H * H; i += blockDim.x) (&w.W2[0][0])[i] = wbf[OFF_W2 + i];
-    for (int i = threadIdx.x; i < H * OUTP; i += blockDim.x) (&w.W3[0][0])[i] = wbf[OFF_W3 + i];
+    static_assert(OFF_W1 % 8 == 0 && OFF_W2 % 8 == 0 && OFF_W3 % 8 == 0, "16-byte rows");
+    auto rows = [&](short* dst, const short* src, int n) {
+        for (int i = threadIdx.x; i < n / 8; i += blockDim.x)
+            reinterpret_cast<int4*>(dst)[i] = reinterpret_cast<const int4*>(src)[i];
+    };
+    rows(&w.W1[0][0], wbf + OFF_W1, INP * H);
+    rows(&w.W2[0][0], wbf + OFF_W2, H * H);
+    rows(&w.W3[0][0], wbf + OFF_W3, H * OUTP);
     for (int i = threadIdx.x; i < H; i += blockDim.x) {
         w.b1[i] = par[OFF_B1 + i];
         w.b2[i] = par[OFF_B2 + i];
@@ -145,14 +151,17 @@ __device__ void forward16(const WeightsLDS& w, WaveLDS& s, const float* __restri
 }
 
 // One wavefront per 16-sample tile (grid-stride); 4 wavefronts per block.
-// grad_slots[wave][NPAR] receives the wave's summed gradient of the mean
-// loss over n samples, loss_slots[wave] its summed loss.
+// grad_slots[block][NPAR] receives the block's summed gradient of the mean loss
+// over n samples (its wavefronts added in order, in LDS: a quarter of the
+// slots to write and to sum), loss_slots[block] its summed loss.
 __global__ void __launch_bounds__(4 * kWave)
 k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const float* __restrict__ feat,
            const int* __restrict__ label, const float* __restrict__ target, int64_t n, float* __restrict__ grad_slots,
            double* __restrict__ loss_slots) {
     __shared__ WeightsLDS w;
     __shared__ WaveLDS wl[4];
+    __shared__ double wave_loss[4];
+    static_assert(sizeof(wl) >= sizeof(float) * NPAR, "the block's gradient takes the tiles' place at the end");
     load_weights(w, wbf, par);
     __syncthreads();
     const int wave = threadIdx.x / kWave;
@@ -251,26 +260,35 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
         for (int m = 0; m < 16; m++) gb1 += bf2f(s.D1[m][lane]);
         __syncthreads();
     }
-    // the wave's slot: C layout element (kq + i, r) of each 16 x 16 tile
-    float* G = grad_slots + gw * (int64_t)NPAR;
+    // the block's gradient: C layout element (kq + i, r) of each 16 x 16 tile
+    float* G = reinterpret_cast<float*>(wl);
+    if (lane == 0) wave_loss[wave] = loss;
+    for (int t = 0; t < 4; t++) {
+        if (wave == t) {
+            auto add = [&](int p, float v) { G[p] = t == 0 ? v : G[p] + v; };
 #pragma unroll
-    for (int nt = 0; nt < H / 16; nt++)
+            for (int nt = 0; nt < H / 16; nt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) G[OFF_W1 + (kq + i) * H + nt * 16 + r] = g1[nt][i];
+                for (int i = 0; i < 4; i++) add(OFF_W1 + (kq + i) * H + nt * 16 + r, g1[nt][i]);
 #pragma unroll
-    for (int mt = 0; mt < H / 16; mt++)
+            for (int mt = 0; mt < H / 16; mt++)
 #pragma unroll
-        for (int nt = 0; nt < H / 16; nt++)
+                for (int nt = 0; nt < H / 16; nt++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) G[OFF_W2 + (mt * 16 + kq + i) * H + nt * 16 + r] = g2[mt][nt][i];
+                    for (int i = 0; i < 4; i++) add(OFF_W2 + (mt * 16 + kq + i) * H + nt * 16 + r, g2[mt][nt][i]);
 #pragma unroll
-    for (int mt = 0; mt < H / 16; mt++)
+            for (int mt = 0; mt < H / 16; mt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) G[OFF_W3 + (mt * 16 + kq + i) * OUTP + r] = g3[mt][i];
-    G[OFF_B1 + lane] = gb1;
-    G[OFF_B2 + lane] = gb2;
-    if (lane < OUTP) G[OFF_B3 + lane] = gb3;
-    if (lane == 0) loss_slots[gw] = loss;
+                for (int i = 0; i < 4; i++) add(OFF_W3 + (mt * 16 + kq + i) * OUTP + r, g3[mt][i]);
+            add(OFF_B1 + lane, gb1);
+            add(OFF_B2 + lane, gb2);
+            if (lane < OUTP) add(OFF_B3 + lane, gb3);
+        }
+        __syncthreads();
+    }
+    float4* out = reinterpret_cast<float4*>(grad_slots + blockIdx.x * (int64_t)NPAR);
+    for (int p = threadIdx.x; p < NPAR / 4; p += 4 * kWave) out[p] = reinterpret_cast<const float4*>(G)[p];
+    if (threadIdx.x == 0) loss_slots[blockIdx.x] = ((wave_loss[0] + wave_loss[1]) + wave_loss[2]) + wave_loss[3];
 }
 
 // Parameters a padded slot never trains: W1 rows >= IN, W3 / b3 columns >= OUT.
@@ -281,15 +299,43 @@ __device__ __forceinline__ bool trainable(int p) {
     return true;
 }
 
-// grad[p] = sum of the slots in slot order; optionally one Adam step.
-__global__ void k_mlp_reduce(const float* __restrict__ slots, int nslots, float* __restrict__ grad,
-                             float* __restrict__ par, float* __restrict__ m1, float* __restrict__ m2,
-                             short* __restrict__ wbf, int adam, float lr, float b1, float b2, float eps, float bc1,
-                             float bc2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPAR) return;
+// grad[p] = sum of the slots -- 16 threads a parameter, each a run of slots in
+// order, then their sums in order -- and optionally one Adam step; block 0
+// leaves the summed loss behind the gradient.  One thread a parameter took
+// 58 us for 256 slots, one load after the other; 64 slots (the block sums of
+// the same minibatch) by 16 threads take 5.
+constexpr int kRedPar = 16, kRedGroups = 16;
+static_assert(NPAR % kRedPar == 0 && NPAR % 4 == 0, "whole blocks, the loss on 8 bytes");
+
+__global__ void __launch_bounds__(kRedPar * kRedGroups)
+k_mlp_reduce(const float* __restrict__ slots, const double* __restrict__ loss_slots, int nslots,
+             float* __restrict__ grad, float* __restrict__ par, float* __restrict__ m1, float* __restrict__ m2,
+             short* __restrict__ wbf, int adam, float lr, float b1, float b2, float eps, float bc1, float bc2) {
+    __shared__ float sums[kRedGroups][kRedPar];
+    __shared__ double losses[kRedPar * kRedGroups];
+    const int t = threadIdx.x, col = t % kRedPar, grp = t / kRedPar;
+    const int p = blockIdx.x * kRedPar + col;
+    const int per = (nslots + kRedGroups - 1) / kRedGroups;
+    const int w0 = min(nslots, grp * per), w1 = min(nslots, w0 + per);
+    float s = 0.f;
+#pragma unroll 4
+    for (int w = w0; w < w1; w++) s += slots[(int64_t)w * NPAR + p];
+    sums[grp][col] = s;
+    if (blockIdx.x == 0) {
+        double l = 0.0;
+        for (int w = t; w < nslots; w += kRedPar * kRedGroups) l += loss_slots[w];
+        losses[t] = l;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && t == 0) {
+        double l = 0.0;
+        for (int i = 0; i < kRedPar * kRedGroups && i < nslots; i++) l += losses[i];
+        *reinterpret_cast<double*>(grad + NPAR) = l;
+    }
+    if (grp != 0) return;
     float g = 0.f;
-    for (int w = 0; w < nslots; w++) g += slots[(int64_t)w * NPAR + p];
+#pragma unroll
+    for (int i = 0; i < kRedGroups; i++) g += sums[i][col];
     if (!trainable(p)) g = 0.f;
     grad[p] = g;
     if (!adam) return;
@@ -463,10 +509,10 @@ void launch_grad(const short* wbf, const float* par, const float* feat, const in
                        loss_slots);
 }
 
-void launch_reduce(const float* slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
+void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
                    bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s) {
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((NPAR + 255) / 256), dim3(256), 0, s, slots, nslots, grad, par, m1, m2, wbf,
-                       adam ? 1 : 0, lr, b1, b2, eps, bc1, bc2);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(NPAR / kRedPar), dim3(kRedPar * kRedGroups), 0, s, slots, loss_slots, nslots,
+                       grad, par, m1, m2, wbf, adam ? 1 : 0, lr, b1, b2, eps, bc1, bc2);
 }
 
 void launch_refresh(const float* par, short* wbf, hipStream_t s) {

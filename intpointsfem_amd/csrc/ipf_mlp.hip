@@ -3,6 +3,7 @@
 // weight copies and gradient slots in device memory).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -24,8 +25,9 @@ struct ipf_mlp {
     float* m1 = nullptr;      // Adam moments
     float* m2 = nullptr;
     short* wbf = nullptr;     // BF16 copies
-    float* grad = nullptr;    // last gradient [NPAR]
-    float* slots = nullptr;   // [kMaxBlocks * 4][NPAR]
+    float* grad = nullptr;    // last gradient [NPAR], then the summed loss (a double)
+    float* host = nullptr;    // pinned copy of the same
+    float* slots = nullptr;   // [kMaxBlocks][NPAR]
     double* loss_slots = nullptr;
     int64_t step = 0;
 };
@@ -106,9 +108,10 @@ int ipf_mlp_create(int device, uint64_t seed, ipf_mlp** out) {
         (rc = hip_check(hipMalloc((void**)&m->m1, sizeof(float) * NPAR), "hipMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->m2, sizeof(float) * NPAR), "hipMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->wbf, sizeof(short) * NPAR), "hipMalloc")) ||
-        (rc = hip_check(hipMalloc((void**)&m->grad, sizeof(float) * NPAR), "hipMalloc")) ||
-        (rc = hip_check(hipMalloc((void**)&m->slots, sizeof(float) * NPAR * 4 * kMaxBlocks), "hipMalloc")) ||
-        (rc = hip_check(hipMalloc((void**)&m->loss_slots, sizeof(double) * 4 * kMaxBlocks), "hipMalloc")))
+        (rc = hip_check(hipMalloc((void**)&m->grad, sizeof(float) * NPAR + sizeof(double)), "hipMalloc")) ||
+        (rc = hip_check(hipHostMalloc((void**)&m->host, sizeof(float) * NPAR + sizeof(double), 0), "hipHostMalloc")) ||
+        (rc = hip_check(hipMalloc((void**)&m->slots, sizeof(float) * NPAR * kMaxBlocks), "hipMalloc")) ||
+        (rc = hip_check(hipMalloc((void**)&m->loss_slots, sizeof(double) * kMaxBlocks), "hipMalloc")))
         return bad(rc);
     m->stream = m->own_stream;
     std::vector<float> p;
@@ -125,6 +128,7 @@ int ipf_mlp_destroy(ipf_mlp* m) {
     for (void* p : {(void*)m->par, (void*)m->m1, (void*)m->m2, (void*)m->wbf, (void*)m->grad, (void*)m->slots,
                     (void*)m->loss_slots})
         if (p) (void)hipFree(p);
+    if (m->host) (void)hipHostFree(m->host);
     if (m->own_stream) (void)hipStreamDestroy(m->own_stream);
     delete m;
     return IPF_OK;
@@ -165,7 +169,7 @@ int ipf_mlp_get_params(ipf_mlp* m, float* params_host) {
 }
 
 static int run_grad(ipf_mlp* m, const float* feat, const int* branch, const float* target, int64_t n, bool adam,
-                    float lr, double* loss) {
+                    float lr, float* grad_host, double* loss) {
     using namespace mlp;
     if (!m || !feat || !branch || !target) return mlp_fail(IPF_EINVAL, "ipf_mlp: NULL argument");
     if (n < 1) return mlp_fail(IPF_EINVAL, "ipf_mlp: need n >= 1 samples");
@@ -179,35 +183,30 @@ static int run_grad(ipf_mlp* m, const float* feat, const int* branch, const floa
         bc1 = 1.f - std::pow(b1, (float)m->step);
         bc2 = 1.f - std::pow(b2, (float)m->step);
     }
-    launch_reduce(m->slots, nb * 4, m->grad, m->par, m->m1, m->m2, m->wbf, adam, lr, b1, b2, 1e-8f, bc1, bc2,
+    launch_reduce(m->slots, m->loss_slots, nb, m->grad, m->par, m->m1, m->m2, m->wbf, adam, lr, b1, b2, 1e-8f, bc1, bc2,
                   m->stream);
     MLP_HIP(hipGetLastError());
-    if (loss) {
-        std::vector<double> ls(nb * 4);
-        MLP_HIP(hipMemcpyAsync(ls.data(), m->loss_slots, sizeof(double) * nb * 4, hipMemcpyDeviceToHost, m->stream));
+    // one copy (of the gradient and the loss behind it, or of the loss) and one wait
+    const int from = grad_host ? 0 : NPAR;
+    if (grad_host || loss) {
+        MLP_HIP(hipMemcpyAsync(m->host + from, m->grad + from, sizeof(float) * (NPAR - from) + sizeof(double),
+                               hipMemcpyDeviceToHost, m->stream));
         MLP_HIP(hipStreamSynchronize(m->stream));
-        double s = 0.0;
-        for (double v : ls) s += v;
-        *loss = s / (double)n;
     }
+    if (grad_host) std::copy(m->host, m->host + NPAR, grad_host);
+    if (loss) *loss = *reinterpret_cast<const double*>(m->host + NPAR) / (double)n;
     return IPF_OK;
 }
 
 int ipf_mlp_gradient(ipf_mlp* m, const float* feat_dev, const int* branch_dev, const float* target_dev, int64_t n,
                      float* grad_host, double* loss) {
-    int rc = run_grad(m, feat_dev, branch_dev, target_dev, n, false, 0.f, loss);
-    if (rc) return rc;
-    if (grad_host) {
-        MLP_HIP(hipMemcpyAsync(grad_host, m->grad, sizeof(float) * mlp::NPAR, hipMemcpyDeviceToHost, m->stream));
-        MLP_HIP(hipStreamSynchronize(m->stream));
-    }
-    return IPF_OK;
+    return run_grad(m, feat_dev, branch_dev, target_dev, n, false, 0.f, grad_host, loss);
 }
 
 int ipf_mlp_train_step(ipf_mlp* m, const float* feat_dev, const int* branch_dev, const float* target_dev, int64_t n,
                        float lr, double* loss) {
     if (!(lr > 0.f)) return mlp_fail(IPF_EINVAL, "ipf_mlp_train_step: need lr > 0");
-    return run_grad(m, feat_dev, branch_dev, target_dev, n, true, lr, loss);
+    return run_grad(m, feat_dev, branch_dev, target_dev, n, true, lr, nullptr, loss);
 }
 
 int ipf_mlp_predict(ipf_mlp* m, const float* feat_dev, int64_t n, int* branch_dev, float* out_dev) {
