@@ -34,11 +34,11 @@ constexpr int NPAR_TRAINABLE = IN * H + H + H * H + H + H * OUT + OUT;  // 5062
 // of NPAR floats) and summed losses (nblocks doubles)
 void launch_grad(const short* wbf, const float* par, const float* feat, const int* label, const float* target,
                  int64_t n, int nblocks, float* slots, double* loss_slots, hipStream_t s);
-// grad = sum of the slots in a fixed order, the summed loss (a double) behind
-// its NPAR floats; with adam, one Adam step on par / m1 / m2
-// (bias corrections bc1 = 1 - b1^t, bc2 = 1 - b2^t) and BF16 copies in wbf
-void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
-                   bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s);
+// grad (or null) = sum of the slots in a fixed order, loss (or null) the summed
+// loss; with adam, one Adam step on par / m1 / m2 (bias corrections bc1 =
+// 1 - b1^t, bc2 = 1 - b2^t) and BF16 copies in wbf
+void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, double* loss, float* par,
+                   float* m1, float* m2, short* wbf, bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s);
 void launch_refresh(const float* par, short* wbf, hipStream_t s);
 void launch_predict(const short* wbf, const float* par, const float* feat, int64_t n, int nblocks, int* branch,
                     float* out, hipStream_t s);

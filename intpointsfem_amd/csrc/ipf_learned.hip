@@ -57,6 +57,7 @@ template <class FA, class FB>
 __device__ __forceinline__ f32x4 mma(FA a, FB b, int K, f32x4 c) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 15, kq = (lane >> 4) * 4;
+#pragma unroll
     for (int k0 = 0; k0 < K; k0 += 16) {
         bf16x4 av, bv;
 #pragma unroll
@@ -218,15 +219,19 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
             for (int j = 0; j < OUTP; j++) s.D3[lane][j] = f2bf(d[j]);
         }
         __syncthreads();
-        if (lane == 0)
+        if (lane == 0) {
+#pragma unroll
             for (int m = 0; m < 16; m++) loss += s.L[m];
+        }
         // layer 3: dW3 += H2^T D3, db3, dZ2 = (D3 W3^T) relu'(Z2)
 #pragma unroll
         for (int mt = 0; mt < H / 16; mt++)
             g3[mt] = mma([&](int m, int k) { return s.H2[k][mt * 16 + m]; }, [&](int k, int j) { return s.D3[k][j]; }, 16,
                          g3[mt]);
-        if (lane < OUTP)
+        if (lane < OUTP) {
+#pragma unroll
             for (int m = 0; m < 16; m++) gb3 += bf2f(s.D3[m][lane]);
+        }
 #pragma unroll
         for (int nt = 0; nt < H / 16; nt++) {
             f32x4 c = {0.f, 0.f, 0.f, 0.f};
@@ -243,6 +248,7 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
             for (int nt = 0; nt < H / 16; nt++)
                 g2[mt][nt] = mma([&](int m, int k) { return s.H1[k][mt * 16 + m]; },
                                  [&](int k, int j) { return s.D2[k][nt * 16 + j]; }, 16, g2[mt][nt]);
+#pragma unroll
         for (int m = 0; m < 16; m++) gb2 += bf2f(s.D2[m][lane]);
 #pragma unroll
         for (int nt = 0; nt < H / 16; nt++) {
@@ -257,6 +263,7 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
         for (int nt = 0; nt < H / 16; nt++)
             g1[nt] = mma([&](int m, int k) { return s.X[k][m]; }, [&](int k, int j) { return s.D1[k][nt * 16 + j]; }, 16,
                          g1[nt]);
+#pragma unroll
         for (int m = 0; m < 16; m++) gb1 += bf2f(s.D1[m][lane]);
         __syncthreads();
     }
@@ -301,16 +308,16 @@ __device__ __forceinline__ bool trainable(int p) {
 
 // grad[p] = sum of the slots -- 16 threads a parameter, each a run of slots in
 // order, then their sums in order -- and optionally one Adam step; block 0
-// leaves the summed loss behind the gradient.  One thread a parameter took
+// sums the loss (grad, loss: where wanted, straight into pinned memory).  One thread a parameter took
 // 58 us for 256 slots, one load after the other; 64 slots (the block sums of
-// the same minibatch) by 16 threads take 5.
+// the same minibatch) by 16 threads take 4.
 constexpr int kRedPar = 16, kRedGroups = 16;
-static_assert(NPAR % kRedPar == 0 && NPAR % 4 == 0, "whole blocks, the loss on 8 bytes");
+static_assert(NPAR % kRedPar == 0 && NPAR % 4 == 0, "whole blocks");
 
 __global__ void __launch_bounds__(kRedPar * kRedGroups)
 k_mlp_reduce(const float* __restrict__ slots, const double* __restrict__ loss_slots, int nslots,
-             float* __restrict__ grad, float* __restrict__ par, float* __restrict__ m1, float* __restrict__ m2,
-             short* __restrict__ wbf, int adam, float lr, float b1, float b2, float eps, float bc1, float bc2) {
+             float* __restrict__ grad, double* __restrict__ loss, float* __restrict__ par, float* __restrict__ m1,
+             float* __restrict__ m2, short* __restrict__ wbf, int adam, float lr, float b1, float b2, float eps, float bc1, float bc2) {
     __shared__ float sums[kRedGroups][kRedPar];
     __shared__ double losses[kRedPar * kRedGroups];
     const int t = threadIdx.x, col = t % kRedPar, grp = t / kRedPar;
@@ -327,17 +334,17 @@ k_mlp_reduce(const float* __restrict__ slots, const double* __restrict__ loss_sl
         losses[t] = l;
     }
     __syncthreads();
-    if (blockIdx.x == 0 && t == 0) {
+    if (loss && blockIdx.x == 0 && t == 0) {
         double l = 0.0;
         for (int i = 0; i < kRedPar * kRedGroups && i < nslots; i++) l += losses[i];
-        *reinterpret_cast<double*>(grad + NPAR) = l;
+        *loss = l;
     }
     if (grp != 0) return;
     float g = 0.f;
 #pragma unroll
     for (int i = 0; i < kRedGroups; i++) g += sums[i][col];
     if (!trainable(p)) g = 0.f;
-    grad[p] = g;
+    if (grad) grad[p] = g;
     if (!adam) return;
     const float a = b1 * m1[p] + (1.f - b1) * g;
     const float v = b2 * m2[p] + (1.f - b2) * g * g;
@@ -509,10 +516,10 @@ void launch_grad(const short* wbf, const float* par, const float* feat, const in
                        loss_slots);
 }
 
-void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, float* par, float* m1, float* m2, short* wbf,
-                   bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s) {
+void launch_reduce(const float* slots, const double* loss_slots, int nslots, float* grad, double* loss, float* par,
+                   float* m1, float* m2, short* wbf, bool adam, float lr, float b1, float b2, float eps, float bc1, float bc2, hipStream_t s) {
     hipLaunchKernelGGL(k_mlp_reduce, dim3(NPAR / kRedPar), dim3(kRedPar * kRedGroups), 0, s, slots, loss_slots, nslots,
-                       grad, par, m1, m2, wbf, adam ? 1 : 0, lr, b1, b2, eps, bc1, bc2);
+                       grad, loss, par, m1, m2, wbf, adam ? 1 : 0, lr, b1, b2, eps, bc1, bc2);
 }
 
 void launch_refresh(const float* par, short* wbf, hipStream_t s) {

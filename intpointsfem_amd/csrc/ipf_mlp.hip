@@ -25,8 +25,7 @@ struct ipf_mlp {
     float* m1 = nullptr;      // Adam moments
     float* m2 = nullptr;
     short* wbf = nullptr;     // BF16 copies
-    float* grad = nullptr;    // last gradient [NPAR], then the summed loss (a double)
-    float* host = nullptr;    // pinned copy of the same
+    float* host = nullptr;    // pinned: the last gradient [NPAR], then the summed loss (a double)
     float* slots = nullptr;   // [kMaxBlocks][NPAR]
     double* loss_slots = nullptr;
     int64_t step = 0;
@@ -108,7 +107,6 @@ int ipf_mlp_create(int device, uint64_t seed, ipf_mlp** out) {
         (rc = hip_check(hipMalloc((void**)&m->m1, sizeof(float) * NPAR), "hipMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->m2, sizeof(float) * NPAR), "hipMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->wbf, sizeof(short) * NPAR), "hipMalloc")) ||
-        (rc = hip_check(hipMalloc((void**)&m->grad, sizeof(float) * NPAR + sizeof(double)), "hipMalloc")) ||
         (rc = hip_check(hipHostMalloc((void**)&m->host, sizeof(float) * NPAR + sizeof(double), 0), "hipHostMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->slots, sizeof(float) * NPAR * kMaxBlocks), "hipMalloc")) ||
         (rc = hip_check(hipMalloc((void**)&m->loss_slots, sizeof(double) * kMaxBlocks), "hipMalloc")))
@@ -125,7 +123,7 @@ int ipf_mlp_destroy(ipf_mlp* m) {
     if (!m) return IPF_OK;
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    for (void* p : {(void*)m->par, (void*)m->m1, (void*)m->m2, (void*)m->wbf, (void*)m->grad, (void*)m->slots,
+    for (void* p : {(void*)m->par, (void*)m->m1, (void*)m->m2, (void*)m->wbf, (void*)m->slots,
                     (void*)m->loss_slots})
         if (p) (void)hipFree(p);
     if (m->host) (void)hipHostFree(m->host);
@@ -183,18 +181,14 @@ static int run_grad(ipf_mlp* m, const float* feat, const int* branch, const floa
         bc1 = 1.f - std::pow(b1, (float)m->step);
         bc2 = 1.f - std::pow(b2, (float)m->step);
     }
-    launch_reduce(m->slots, m->loss_slots, nb, m->grad, m->par, m->m1, m->m2, m->wbf, adam, lr, b1, b2, 1e-8f, bc1, bc2,
-                  m->stream);
+    // what the caller wants goes straight into pinned memory: one wait, no copy
+    double* hloss = reinterpret_cast<double*>(m->host + NPAR);
+    launch_reduce(m->slots, m->loss_slots, nb, grad_host ? m->host : nullptr, loss ? hloss : nullptr, m->par, m->m1, m->m2,
+                  m->wbf, adam, lr, b1, b2, 1e-8f, bc1, bc2, m->stream);
     MLP_HIP(hipGetLastError());
-    // one copy (of the gradient and the loss behind it, or of the loss) and one wait
-    const int from = grad_host ? 0 : NPAR;
-    if (grad_host || loss) {
-        MLP_HIP(hipMemcpyAsync(m->host + from, m->grad + from, sizeof(float) * (NPAR - from) + sizeof(double),
-                               hipMemcpyDeviceToHost, m->stream));
-        MLP_HIP(hipStreamSynchronize(m->stream));
-    }
+    if (grad_host || loss) MLP_HIP(hipStreamSynchronize(m->stream));
     if (grad_host) std::copy(m->host, m->host + NPAR, grad_host);
-    if (loss) *loss = *reinterpret_cast<const double*>(m->host + NPAR) / (double)n;
+    if (loss) *loss = *hloss / (double)n;
     return IPF_OK;
 }
 
