@@ -74,6 +74,15 @@ struct WaveSum {
 };
 __device__ __forceinline__ double cg_beta(double rz, double rz_old) { return rz_old != 0.0 ? rz / rz_old : 0.0; }
 
+// Orders the LDS accesses of one wavefront (its lanes exchange values
+// through LDS; LDS instructions of a wavefront execute in order, so only
+// the compiler must not move them across this point).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct PointState {
     const double* w;
     double* ep0;          // plastic strain XX

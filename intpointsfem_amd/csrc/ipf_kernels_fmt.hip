@@ -419,15 +419,6 @@ __global__ void k_build_B(GroupDev g, const double* __restrict__ corners, double
     w[g.pt0 + tile * C::TP + lane] = wt;
 }
 
-// Orders the LDS accesses of one wavefront (its lanes exchange values
-// through LDS; LDS instructions of a wavefront execute in order, so only
-// the compiler must not move them across this point).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The non-committing residual over the patch layout (ipf_patch.h): one
 // workgroup of NW wavefronts per patch.  Per point the
 // colored kernel's arithmetic (geometric FP64 B, compact strain sums, return

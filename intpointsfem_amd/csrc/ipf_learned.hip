@@ -52,38 +52,6 @@ __device__ __forceinline__ float bf2f(short h) { return __uint_as_float(((uint32
 __device__ __forceinline__ float relu(float x) { return __int_as_float(max(__float_as_int(x), 0)); }
 __device__ __forceinline__ float relu_grad(float x) { return x > 0.f ? 1.f : 0.f; }
 
-// C += A (16 x K) B (K x 16); a(m, k), b(k, n) return BF16 bits.
-template <class FA, class FB>
-__device__ __forceinline__ f32x4 mma(FA a, FB b, int K, f32x4 c) {
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-#pragma unroll
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        bf16x4 av, bv;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            av[i] = a(r, k0 + kq + i);
-            bv[i] = b(k0 + kq + i, r);
-        }
-        c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, c, 0, 0, 0);
-    }
-    return c;
-}
-
-// Per-wavefront LDS of the forward / backward pass over 16 samples.
-struct WaveLDS {
-    short X[16][INP];       // inputs (BF16)
-    float Z1[16][H];        // pre-activations (FP32)
-    float Z2[16][H];
-    short H1[16][H];        // activations (BF16)
-    short H2[16][H];
-    float Z3[16][OUTP];     // outputs
-    short D3[16][OUTP];     // dL/dZ3 (BF16)
-    short D2[16][H];        // dL/dZ2
-    short D1[16][H];        // dL/dZ1
-    float L[16];            // per-sample loss
-};
-
 struct WeightsLDS {
     alignas(16) short W1[INP][H];
     alignas(16) short W2[H][H];
@@ -108,167 +76,224 @@ __device__ void load_weights(WeightsLDS& w, const short* __restrict__ wbf, const
     for (int i = threadIdx.x; i < OUTP; i += blockDim.x) w.b3[i] = par[OFF_B3 + i];
 }
 
-// forward pass of the wave's 16 samples starting at s0 (rows >= n are zero)
-__device__ void forward16(const WeightsLDS& w, WaveLDS& s, const float* __restrict__ feat, int64_t s0, int64_t n) {
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    for (int t = lane; t < 16 * INP; t += kWave) {
-        const int m = t / INP, k = t - m * INP;
-        const int64_t q = s0 + m;
-        s.X[m][k] = (k < IN && q < n) ? f2bf(feat[q * FEAT_STRIDE + k]) : (short)0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int nt = 0; nt < H / 16; nt++) {
-        f32x4 c = {0.f, 0.f, 0.f, 0.f};
-        c = mma([&](int m, int k) { return s.X[m][k]; }, [&](int k, int j) { return w.W1[k][nt * 16 + j]; }, INP, c);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float z = c[i] + w.b1[nt * 16 + r];
-            s.Z1[kq + i][nt * 16 + r] = z;
-            s.H1[kq + i][nt * 16 + r] = f2bf(relu(z));
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int nt = 0; nt < H / 16; nt++) {
-        f32x4 c = {0.f, 0.f, 0.f, 0.f};
-        c = mma([&](int m, int k) { return s.H1[m][k]; }, [&](int k, int j) { return w.W2[k][nt * 16 + j]; }, H, c);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float z = c[i] + w.b2[nt * 16 + r];
-            s.Z2[kq + i][nt * 16 + r] = z;
-            s.H2[kq + i][nt * 16 + r] = f2bf(relu(z));
-        }
-    }
-    __syncthreads();
-    {
-        f32x4 c = {0.f, 0.f, 0.f, 0.f};
-        c = mma([&](int m, int k) { return s.H2[m][k]; }, [&](int k, int j) { return w.W3[k][j]; }, H, c);
-#pragma unroll
-        for (int i = 0; i < 4; i++) s.Z3[kq + i][r] = c[i] + w.b3[r];
-    }
-    __syncthreads();
+typedef __bf16 bf16x4_hw __attribute__((ext_vector_type(4)));
+
+// Four FP32 values to BF16 with the hardware conversion (v_cvt_pk_bf16_f32:
+// round to nearest even, f2bf's result for every finite value).
+__device__ __forceinline__ bf16x4 to_bf16x4(f32x4 v) {
+    return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, bf16x4_hw));
 }
+
+// C += A B over one K step of 16
+__device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 relu4(f32x4 z) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) z[i] = relu(z[i]);
+    return z;
+}
+
+// c relu'(z)
+__device__ __forceinline__ f32x4 relu_grad4(f32x4 c, f32x4 z) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) c[i] = c[i] * relu_grad(z[i]);
+    return c;
+}
+
+__device__ __forceinline__ float sum_bf4(bf16x4 v) { return ((bf2f(v[0]) + bf2f(v[1])) + bf2f(v[2])) + bf2f(v[3]); }
 
 // One wavefront per 16-sample tile (grid-stride); 4 wavefronts per block.
 // grad_slots[block][NPAR] receives the block's summed gradient of the mean loss
 // over n samples (its wavefronts added in order, in LDS: a quarter of the
 // slots to write and to sum), loss_slots[block] its summed loss.
+//
+// Activations stay in registers.  A C fragment of a transposed product (Z^T:
+// lane = sample + 16 (unit / 4), value unit % 4) is an operand of the next
+// product over those units, and one of the plain product (Z: lane = unit + 16
+// (sample / 4), value sample % 4) is an operand of a weight gradient, a product
+// over the samples; the two products take the same operand registers, swapped.
+// So each layer is multiplied twice (92 MFMAs a tile) and nothing passes
+// through LDS but the 16 x 16 output derivatives, turned once -- against two
+// LDS bytes per value and eight 2-byte LDS reads per MFMA before.  Gradient call
+// (with the sums): 4,096 samples 38 -> 32 us (bound by two launches and the
+// weights' way into registers), 500,000 with the sums as they were before 642
+// -> 116, 2 million 1,676 -> 353.
 __global__ void __launch_bounds__(4 * kWave)
 k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const float* __restrict__ feat,
            const int* __restrict__ label, const float* __restrict__ target, int64_t n, float* __restrict__ grad_slots,
            double* __restrict__ loss_slots) {
+    constexpr int NT = H / 16;
     __shared__ WeightsLDS w;
-    __shared__ WaveLDS wl[4];
+    __shared__ float G[NPAR];
+    __shared__ short turn[4][16][OUTP];
     __shared__ double wave_loss[4];
-    static_assert(sizeof(wl) >= sizeof(float) * NPAR, "the block's gradient takes the tiles' place at the end");
     load_weights(w, wbf, par);
     __syncthreads();
     const int wave = threadIdx.x / kWave;
     const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    WaveLDS& s = wl[wave];
-    const int64_t gw = (int64_t)blockIdx.x * 4 + wave;
+    const int r = lane & 15, g = lane >> 4, kq = g * 4;
+    // weight operands: rows over the inputs (w1, w2, w3), over the outputs (v2, v3)
+    bf16x4 w1[NT], w2[NT][NT], w3[NT], v2[NT][NT], v3[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            w1[t][i] = w.W1[kq + i][16 * t + r];
+            w3[t][i] = w.W3[16 * t + kq + i][r];
+            v3[t][i] = w.W3[16 * t + r][kq + i];
+#pragma unroll
+            for (int u = 0; u < NT; u++) {
+                w2[u][t][i] = w.W2[16 * t + kq + i][16 * u + r];
+                v2[t][u][i] = w.W2[16 * t + r][16 * u + kq + i];
+            }
+        }
+    }
     const int64_t nw = (int64_t)gridDim.x * 4;
     const int64_t ntile = (n + 15) / 16;
     const float inv_n = 1.f / (float)n;
-    f32x4 g1[H / 16], g2[H / 16][H / 16], g3[H / 16];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 g1[NT], g2[NT][NT], g3[NT];
+    float gb1[NT], gb2[NT], gb3 = 0.f;  // lane (r, g): column r of tile t, samples 4g..4g+3
 #pragma unroll
-    for (int a = 0; a < H / 16; a++) {
-        g1[a] = g3[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int a = 0; a < NT; a++) {
+        g1[a] = g3[a] = zero;
+        gb1[a] = gb2[a] = 0.f;
 #pragma unroll
-        for (int b = 0; b < H / 16; b++) g2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < NT; b++) g2[a][b] = zero;
     }
-    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f;  // lane j: bias column j
     double loss = 0.0;
-    // every wavefront runs the same number of rounds, so the block barriers
-    // inside forward16 / the backward are reached by all four
-    const int64_t rounds = (ntile + nw - 1) / nw;
-    for (int64_t rd = 0; rd < rounds; rd++) {
-        const int64_t tile = rd * nw + gw;
-        const int64_t s0 = tile * 16;
-        forward16(w, s, feat, s0, n);
-        // loss and dL/dZ3 per sample (lanes 0..15 own one sample each)
-        if (lane < 16) {
-            const int64_t q = s0 + lane;
-            float d[OUTP];
+    for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < ntile; tile += nw) {
+        const int64_t s0 = tile * 16, q = s0 + r;
+        // inputs: features 4g.. of sample r, and feature r of samples 4g..
+        f32x4 xf = zero, xs = zero;
+        if (g < 2 && q < n) xf = *reinterpret_cast<const f32x4*>(feat + q * FEAT_STRIDE + 4 * g);
+        if (g == 1) xf[3] = 0.f;  // IN = 7 features
 #pragma unroll
-            for (int j = 0; j < OUTP; j++) d[j] = 0.f;
-            float l = 0.f;
-            if (q < n) {
-                float zmax = s.Z3[lane][0];
+        for (int i = 0; i < 4; i++)
+            if (r < IN && s0 + kq + i < n) xs[i] = feat[(s0 + kq + i) * FEAT_STRIDE + r];
+        const int y = q < n ? label[q] : 0;
+        const float tg = q < n ? target[q] : 0.f;
+        const bf16x4 xb = to_bf16x4(xf), xt = to_bf16x4(xs);
+        // layer 1: Z1^T and Z1
+        bf16x4 h1t[NT], h1n[NT];
+        f32x4 z1n[NT];
 #pragma unroll
-                for (int j = 1; j < NBR; j++) zmax = fmaxf(zmax, s.Z3[lane][j]);
-                float e[NBR], se = 0.f;
+        for (int t = 0; t < NT; t++) {
+            f32x4 z = mfma16(w1[t], xb, zero);
 #pragma unroll
-                for (int j = 0; j < NBR; j++) {
-                    e[j] = expf(s.Z3[lane][j] - zmax);
-                    se += e[j];
-                }
-                const int y = label[q];
-                l = -(s.Z3[lane][y] - zmax - logf(se));
+            for (int i = 0; i < 4; i++) z[i] = z[i] + w.b1[16 * t + kq + i];
+            h1t[t] = to_bf16x4(relu4(z));
+            z1n[t] = mfma16(xb, w1[t], zero);
+            const float b = w.b1[16 * t + r];
 #pragma unroll
-                for (int j = 0; j < NBR; j++) d[j] = (e[j] / se - (j == y ? 1.f : 0.f)) * inv_n;
-                const float diff = s.Z3[lane][NBR] - target[q];
-                l += REG_WEIGHT * diff * diff;
-                d[NBR] = 2.f * REG_WEIGHT * diff * inv_n;
+            for (int i = 0; i < 4; i++) z1n[t][i] = z1n[t][i] + b;
+            h1n[t] = to_bf16x4(relu4(z1n[t]));
+        }
+        // layer 2
+        bf16x4 h2t[NT], h2n[NT];
+        f32x4 z2t[NT], z2n[NT];
+#pragma unroll
+        for (int u = 0; u < NT; u++) {
+            f32x4 a = zero, b = zero;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                a = mfma16(w2[u][t], h1t[t], a);
+                b = mfma16(h1t[t], w2[u][t], b);
             }
-            s.L[lane] = l;
+            const float bias = w.b2[16 * u + r];
 #pragma unroll
-            for (int j = 0; j < OUTP; j++) s.D3[lane][j] = f2bf(d[j]);
+            for (int i = 0; i < 4; i++) {
+                a[i] = a[i] + w.b2[16 * u + kq + i];
+                b[i] = b[i] + bias;
+            }
+            z2t[u] = a;
+            z2n[u] = b;
+            h2t[u] = to_bf16x4(relu4(a));
+            h2n[u] = to_bf16x4(relu4(b));
         }
-        __syncthreads();
-        if (lane == 0) {
+        // layer 3: Z3^T, lane (r, g) holds outputs 4g.. of sample r
+        f32x4 o = zero;
 #pragma unroll
-            for (int m = 0; m < 16; m++) loss += s.L[m];
+        for (int t = 0; t < NT; t++) o = mfma16(w3[t], h2t[t], o);
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] = o[i] + w.b3[kq + i];
+        // loss and dL/dZ3: every lane of a sample has its six outputs
+        float z[OUT];
+#pragma unroll
+        for (int j = 0; j < 4; j++) z[j] = __shfl(o[j], r, kWave);
+        z[4] = __shfl(o[0], r + 16, kWave);
+        z[5] = __shfl(o[1], r + 16, kWave);
+        float zmax = z[0];
+#pragma unroll
+        for (int j = 1; j < NBR; j++) zmax = fmaxf(zmax, z[j]);
+        float e[NBR], se = 0.f, zy = z[0];
+#pragma unroll
+        for (int j = 0; j < NBR; j++) {
+            e[j] = expf(z[j] - zmax);
+            se += e[j];
+            if (j == y) zy = z[j];
         }
-        // layer 3: dW3 += H2^T D3, db3, dZ2 = (D3 W3^T) relu'(Z2)
+        const float diff = z[NBR] - tg;
+        f32x4 d = zero;
+        if (q < n) {
+            if (g == 0) {
 #pragma unroll
-        for (int mt = 0; mt < H / 16; mt++)
-            g3[mt] = mma([&](int m, int k) { return s.H2[k][mt * 16 + m]; }, [&](int k, int j) { return s.D3[k][j]; }, 16,
-                         g3[mt]);
-        if (lane < OUTP) {
-#pragma unroll
-            for (int m = 0; m < 16; m++) gb3 += bf2f(s.D3[m][lane]);
+                for (int j = 0; j < 4; j++) d[j] = (e[j] / se - (j == y ? 1.f : 0.f)) * inv_n;
+                float l = -(zy - zmax - logf(se));
+                l += REG_WEIGHT * diff * diff;
+                loss += l;
+            } else if (g == 1) {
+                d[0] = (e[4] / se - (4 == y ? 1.f : 0.f)) * inv_n;
+                d[1] = 2.f * REG_WEIGHT * diff * inv_n;
+            }
         }
+        const bf16x4 d3t = to_bf16x4(d);
+        *reinterpret_cast<bf16x4*>(&turn[wave][r][kq]) = d3t;
+        wave_lds_sync();
+        bf16x4 d3n;
 #pragma unroll
-        for (int nt = 0; nt < H / 16; nt++) {
-            f32x4 c = {0.f, 0.f, 0.f, 0.f};
-            c = mma([&](int m, int k) { return s.D3[m][k]; }, [&](int k, int j) { return w.W3[nt * 16 + j][k]; }, OUTP,
-                    c);
+        for (int i = 0; i < 4; i++) d3n[i] = turn[wave][kq + i][r];
+        wave_lds_sync();
+        gb3 += sum_bf4(d3n);
+        // layer 2's derivatives, both ways; dW3 += H2^T D3
+        bf16x4 d2t[NT], d2n[NT];
 #pragma unroll
-            for (int i = 0; i < 4; i++) s.D2[kq + i][nt * 16 + r] = f2bf(c[i] * relu_grad(s.Z2[kq + i][nt * 16 + r]));
+        for (int u = 0; u < NT; u++) {
+            g3[u] = mfma16(h2n[u], d3n, g3[u]);
+            d2t[u] = to_bf16x4(relu_grad4(mfma16(v3[u], d3t, zero), z2t[u]));
+            d2n[u] = to_bf16x4(relu_grad4(mfma16(d3t, v3[u], zero), z2n[u]));
+            gb2[u] += sum_bf4(d2n[u]);
         }
-        __syncthreads();
-        // layer 2: dW2 += H1^T D2, db2, dZ1 = (D2 W2^T) relu'(Z1)
+        // dW2 += H1^T D2; D1 and dW1 += X^T D1
 #pragma unroll
-        for (int mt = 0; mt < H / 16; mt++)
+        for (int t = 0; t < NT; t++) {
+            f32x4 c = zero;
 #pragma unroll
-            for (int nt = 0; nt < H / 16; nt++)
-                g2[mt][nt] = mma([&](int m, int k) { return s.H1[k][mt * 16 + m]; },
-                                 [&](int k, int j) { return s.D2[k][nt * 16 + j]; }, 16, g2[mt][nt]);
-#pragma unroll
-        for (int m = 0; m < 16; m++) gb2 += bf2f(s.D2[m][lane]);
-#pragma unroll
-        for (int nt = 0; nt < H / 16; nt++) {
-            f32x4 c = {0.f, 0.f, 0.f, 0.f};
-            c = mma([&](int m, int k) { return s.D2[m][k]; }, [&](int k, int j) { return w.W2[nt * 16 + j][k]; }, H, c);
-#pragma unroll
-            for (int i = 0; i < 4; i++) s.D1[kq + i][nt * 16 + r] = f2bf(c[i] * relu_grad(s.Z1[kq + i][nt * 16 + r]));
+            for (int u = 0; u < NT; u++) {
+                g2[t][u] = mfma16(h1n[t], d2n[u], g2[t][u]);
+                c = mfma16(d2t[u], v2[t][u], c);
+            }
+            const bf16x4 d1n = to_bf16x4(relu_grad4(c, z1n[t]));
+            gb1[t] += sum_bf4(d1n);
+            g1[t] = mfma16(xt, d1n, g1[t]);
         }
-        __syncthreads();
-        // layer 1: dW1 += X^T D1, db1
-#pragma unroll
-        for (int nt = 0; nt < H / 16; nt++)
-            g1[nt] = mma([&](int m, int k) { return s.X[k][m]; }, [&](int k, int j) { return s.D1[k][nt * 16 + j]; }, 16,
-                         g1[nt]);
-#pragma unroll
-        for (int m = 0; m < 16; m++) gb1 += bf2f(s.D1[m][lane]);
-        __syncthreads();
     }
+    // the columns' four sample groups, the samples' losses
+    auto over_groups = [&](float v) {
+        v += __shfl_xor(v, 16, kWave);
+        return v + __shfl_xor(v, 32, kWave);
+    };
+    gb3 = over_groups(gb3);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        gb1[t] = over_groups(gb1[t]);
+        gb2[t] = over_groups(gb2[t]);
+    }
+#pragma unroll
+    for (int k = 8; k > 0; k >>= 1) loss += __shfl_xor(loss, k, kWave);  // lanes 0..15 hold them
     // the block's gradient: C layout element (kq + i, r) of each 16 x 16 tile
-    float* G = reinterpret_cast<float*>(wl);
     if (lane == 0) wave_loss[wave] = loss;
     for (int t = 0; t < 4; t++) {
         if (wave == t) {
@@ -287,9 +312,14 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
             for (int mt = 0; mt < H / 16; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) add(OFF_W3 + (mt * 16 + kq + i) * OUTP + r, g3[mt][i]);
-            add(OFF_B1 + lane, gb1);
-            add(OFF_B2 + lane, gb2);
-            if (lane < OUTP) add(OFF_B3 + lane, gb3);
+            if (g == 0) {
+#pragma unroll
+                for (int u = 0; u < NT; u++) {
+                    add(OFF_B1 + 16 * u + r, gb1[u]);
+                    add(OFF_B2 + 16 * u + r, gb2[u]);
+                }
+                add(OFF_B3 + r, gb3);
+            }
         }
         __syncthreads();
     }
@@ -359,14 +389,6 @@ k_mlp_reduce(const float* __restrict__ slots, const double* __restrict__ loss_sl
 __global__ void k_mlp_refresh(const float* __restrict__ par, short* __restrict__ wbf) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p < NPAR) wbf[p] = f2bf(par[p]);
-}
-
-typedef __bf16 bf16x4_hw __attribute__((ext_vector_type(4)));
-
-// Four FP32 values to BF16 with the hardware conversion (v_cvt_pk_bf16_f32:
-// round to nearest even, f2bf's result for every finite value).
-__device__ __forceinline__ bf16x4 to_bf16x4(f32x4 v) {
-    return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, bf16x4_hw));
 }
 
 // C += A B over 32 k with gfx950's 16 x 16 x 32 BF16 MFMA, the operands two
