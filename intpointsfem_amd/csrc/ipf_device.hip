@@ -763,18 +763,21 @@ void build_split(ipf_ctx* ctx) {
     for (int sh = 0; sh < SHAPE_COUNT; sh++) {
         SplitDev& d = ctx->split[sh];
         d = SplitDev{};
-        const int ET = shape_et(sh), NE = ET * (shape_ce(sh) / 2), TP = shape_tp(sh);
         for (const auto& g : ctx->groups) {
             if (g.shape != sh) continue;
-            const int64_t t0 = d.ntiles;  // launch tile of the group's first
-            d.tile0[d.nseg] = (int)(g.tile0 - t0);
-            d.pt0[d.nseg] = (int)(g.pt0 - t0 * TP);
-            d.slot0[d.nseg] = (int)(g.slot0 - t0 * ET);
-            d.ent0[d.nseg] = (int)(g.dof_off / 2 - t0 * NE);
-            d.val0[d.nseg] = g.f_off[FMT_C64] - t0 * format_values(sh, FMT_C64) * TP;
+            d.count[d.nseg] = (int)g.ntiles;
+            d.tile0[d.nseg] = (int)g.tile0;
+            d.pt0[d.nseg] = (int)g.pt0;
+            d.slot0[d.nseg] = (int)g.slot0;
+            d.ent0[d.nseg] = (int)(g.dof_off / 2);
+            d.val0[d.nseg] = g.f_off[FMT_C64];
+            d.even = d.nseg ? std::min(d.even, d.count[d.nseg]) : d.count[d.nseg];
             d.ntiles += g.ntiles;
-            d.end[d.nseg++] = (int)d.ntiles;
+            d.nseg++;
         }
+        // t / 1 by mulhi would need 2^32: one segment is all rest
+        d.magic = d.nseg > 1 ? (unsigned)((0x100000000ull + d.nseg - 1) / d.nseg) : 0xffffffffu;
+        if (d.nseg == 1) d.even = 0;
         d.tmeta = ctx->dTmeta;
         d.node = ctx->dNodeR;
     }

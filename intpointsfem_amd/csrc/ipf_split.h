@@ -11,12 +11,17 @@ namespace ipf {
 constexpr int kSplitColors = 8;  // colors (and so groups of one shape) at most
 
 // One element launch: the tiles of one shape, every color.  Segment c is the
-// shape's group of one color: launch tiles [end[c - 1], end[c]), and where its
-// tile 0 would start if the group began at launch tile 0 -- so that a tile's
-// addresses follow from its number without a load.
+// shape's group of one color, `count` tiles; launch tile t is tile t / nseg of
+// segment t mod nseg while every segment has one (t < even nseg), then what is
+// left segment by segment.  Neighbouring elements of different colors so run
+// side by side on one XCD, whose L2 holds the lines they share -- u, and rows
+// of per-point values in the reference order -- and a tile's addresses follow
+// from its number without a load.
 struct SplitDev {
     int nseg;
-    int end[kSplitColors];
+    int even;                     // the smallest segment's tiles
+    unsigned magic;               // ceil(2^32 / nseg): t / nseg = mulhi(t, magic) for t < 2^29
+    int count[kSplitColors];
     int tile0[kSplitColors];      // context tile (tmeta)
     int pt0[kSplitColors];        // new point
     int slot0[kSplitColors];      // element slot (corners)

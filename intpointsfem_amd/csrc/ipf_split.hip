@@ -15,6 +15,24 @@ namespace ipf {
 
 namespace {
 
+// Segment and tile inside it of launch tile t (SplitDev).
+struct SplitTile {
+    int seg, t;
+};
+
+__device__ __forceinline__ SplitTile split_tile(const SplitDev& g, int t) {
+    const int q = (int)__umulhi((unsigned)t, g.magic);
+    if (q < g.even) return SplitTile{t - q * g.nseg, q};
+    int rest = t - g.even * g.nseg, seg = 0;
+#pragma unroll
+    for (int c = 0; c < kSplitColors - 1; c++)
+        if (c == seg && rest >= g.count[c] - g.even) {
+            rest -= g.count[c] - g.even;
+            seg = c + 1;
+        }
+    return SplitTile{seg, g.even + rest};
+}
+
 // Values of the tile's points, N each, between LDS (point order) and the
 // reference order: an element's points are consecutive there, so the
 // wavefront reads and writes whole rows of it (lane by lane it would touch
@@ -64,12 +82,13 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     __shared__ double pts[POINTS ? 3 * C::TP : 1];
     __shared__ int64_t oel[POINTS ? C::ET : 1];
     const int lane = threadIdx.x;
-    const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const SplitTile at = split_tile(g, (int)xcd_tile(blockIdx.x, gridDim.x));
+    const int t = at.t;
     int tile0 = g.tile0[0], pt0 = g.pt0[0], slot0 = g.slot0[0], ent0 = g.ent0[0];
     int64_t val0 = g.val0[0];
 #pragma unroll
     for (int c = 1; c < kSplitColors; c++)
-        if (c < g.nseg && t >= g.end[c - 1]) {
+        if (c == at.seg) {
             tile0 = g.tile0[c];
             pt0 = g.pt0[c];
             slot0 = g.slot0[c];
@@ -245,11 +264,12 @@ k_stress(SplitDev g, const double* __restrict__ strain, double* __restrict__ wsi
     __shared__ double sh[N * TP];
     __shared__ int64_t oel[ET];
     const int lane = threadIdx.x;
-    const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const SplitTile at = split_tile(g, (int)xcd_tile(blockIdx.x, gridDim.x));
+    const int t = at.t;
     int tile0 = g.tile0[0], pt0 = g.pt0[0];
 #pragma unroll
     for (int c = 1; c < kSplitColors; c++)
-        if (c < g.nseg && t >= g.end[c - 1]) {
+        if (c == at.seg) {
             tile0 = g.tile0[c];
             pt0 = g.pt0[c];
         }
