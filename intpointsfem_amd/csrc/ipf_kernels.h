@@ -72,6 +72,19 @@ struct WaveSum {
         return s;
     }
 };
+// The sum over a block of NW wavefronts, valid in thread 0: lanes by shuffles,
+// then the wavefronts in order (one barrier; sh: NW doubles).
+template <int NW>
+__device__ __forceinline__ double block_sum_waves(double v, double* sh) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = sh[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) s = s + sh[w];
+    return s;
+}
 __device__ __forceinline__ double cg_beta(double rz, double rz_old) { return rz_old != 0.0 ? rz / rz_old : 0.0; }
 
 // Orders the LDS accesses of one wavefront (its lanes exchange values

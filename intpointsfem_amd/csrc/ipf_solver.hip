@@ -150,7 +150,7 @@ k_cg_update_dot(int64_t n, const double* __restrict__ rz_new, const double* __re
                 const double* __restrict__ p, const double* __restrict__ q, double* __restrict__ x,
                 double* __restrict__ r, const double* __restrict__ pa, const double* __restrict__ pb,
                 double* __restrict__ z, double* __restrict__ partial, double* __restrict__ rr_partial) {
-    __shared__ double sh[kDotThreads];
+    __shared__ double sh[2][kDotThreads / 64];
     double s = 0.0, rr = 0.0;
     // one DoF pair per thread and step (see k_cg_init); batches of U whole
     // pairs with every load in flight at once, then the same arithmetic and
@@ -253,11 +253,10 @@ k_cg_update_dot(int64_t n, const double* __restrict__ rz_new, const double* __re
         }
         if (RR) rr = (rr + r0 * r0) + r1 * r1;
     }
-    const double t = block_sum(s, sh);
+    const double t = block_sum_waves<kDotThreads / 64>(s, sh[0]);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
     if (RR) {
-        __syncthreads();
-        const double t2 = block_sum(rr, sh);
+        const double t2 = block_sum_waves<kDotThreads / 64>(rr, sh[1]);
         if (threadIdx.x == 0) rr_partial[blockIdx.x] = t2;
     }
 }

@@ -386,7 +386,7 @@ __global__ void __launch_bounds__(256)
 k_nodes_cg(int64_t n, const int* __restrict__ map, const dv2* __restrict__ ef, const signed char* __restrict__ mask,
            const double* __restrict__ z, CgBeta cg, double* __restrict__ rz_new, double* __restrict__ p,
            double* __restrict__ q, double* __restrict__ partial) {
-    __shared__ double sh[256];
+    __shared__ double sh[4];
     double s = 0.0, beta = 0.0;
     // the first node's requests leave with those of beta
     const WaveSum ws(cg.nrz, cg.rz_partial);
@@ -423,13 +423,8 @@ k_nodes_cg(int64_t n, const int* __restrict__ map, const dv2* __restrict__ ef, c
             }
         }
     }
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
+    const double sum = block_sum_waves<4>(s, sh);
+    if (threadIdx.x == 0) partial[blockIdx.x] = sum;
 }
 
 template <int FMT, int OP>
