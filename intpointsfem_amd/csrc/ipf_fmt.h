@@ -164,6 +164,27 @@ constexpr int row_stride(int w, int bytes) {
     return (q % 2 ? q : q + 1) * per;
 }
 
+// The element launch of the residual with tangent parks B in LDS while the
+// return map and the tangent fill the registers (a row of the lane's own, read
+// back before the rows are staged): two wavefronts per SIMD at Q2 become three
+// at 140 VGPRs; residual, tangent and K of 201x150 Q2 74 us, so 71 to 72.  Not at
+// Q1, which has three anyway, nor at Q3, whose rows would take 17 KB per
+// wavefront, nor in the launch per color, which spills at three (400x400 Q2
+// 148 us, so 184).
+constexpr bool park_B(int ce) { return ce > 8 && ce <= 20; }
+template <int N, class T>
+__device__ __forceinline__ void park(T* row, const T* b) {
+#pragma unroll
+    for (int k = 0; k < N; k++) row[k] = b[k];
+    asm volatile("" ::: "memory");  // read back, not kept
+}
+template <int N, class T>
+__device__ __forceinline__ void unpark(const T* row, T* b) {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int k = 0; k < N; k++) b[k] = row[k];
+}
+
 // Columns [J0, J1) of one point's B^T (w sigma) partials into row[j - J0].
 // Dense: rows summed in order per column; compact: the same sums without the
 // zero terms.  The residual and tangent kernels stage half the columns at a

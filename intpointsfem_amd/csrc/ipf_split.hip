@@ -62,7 +62,7 @@ __device__ __forceinline__ void load_points(double* sh, const int64_t* oel, int 
 // and last round trip (a product with w Dep requested after the gather and
 // the addresses read from a table: 20x20 Q2 7.8 us, so 6.3).
 template <int SHAPE, int FMT, int OP>
-__global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 8 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
+__global__ void __launch_bounds__(kWave, (OP == EL_DEP ? (FC<SHAPE, FMT>::CE <= 20 ? 3 : 2) : FC<SHAPE, FMT>::MIN_WAVES))
 k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     using C = FC<SHAPE, FMT>;
     using T = typename C::T;
@@ -77,7 +77,9 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     constexpr int RS = row_stride(H, sizeof(T)), RS2 = row_stride(H2, sizeof(T));
     constexpr int NE = C::ET * NSH;
     static_assert(NE <= kWave, "one node per lane");
-    __shared__ T lds[FORCES ? C::TP * (RS > RS2 ? RS : RS2) : 1];
+    constexpr bool PARK = OP == EL_DEP && park_B(C::CE);
+    constexpr int PS = PARK ? row_stride(C::NV, sizeof(T)) : 0;
+    __shared__ T lds[FORCES ? C::TP * (PARK ? PS : RS > RS2 ? RS : RS2) : 1];
     __shared__ double us[GATHER ? 2 * NE : 1];
     __shared__ double pts[POINTS ? 3 * C::TP : 1];
     __shared__ int64_t oel[POINTS ? C::ET : 1];
@@ -173,6 +175,7 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
     if (valid) {
         double e3[3];
         if constexpr (GATHER) strain_fmt<SHAPE, FMT>(b, us + el * C::CE, e3);
+        if (PARK) park<C::NV>(lds + lane * PS, b);
         if constexpr (OP == EL_STRAIN) {
 #pragma unroll
             for (int k = 0; k < 3; k++) pts[3 * lane + k] = e3[k];
@@ -204,6 +207,7 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
                 point_sigma<true>(e3, ep, alpha, mt, br, mc, w, x, d9);
 #pragma unroll
                 for (int k = 0; k < 9; k++) a.dep[k * a.npad + P] = d9[k];
+                if (PARK) unpark<C::NV>(lds + lane * PS, b);
             } else if (!(OP == EL_CERTIFIED && certified_elastic(e3, ep, mc, w, x))) {
                 int mt, br;
                 point_sigma<false>(e3, ep, alpha, mt, br, mc, w, x, nullptr);
@@ -215,6 +219,7 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
         store_points<3, C::NIP>(pts, oel, nv, a.point);
     }
     if constexpr (!FORCES) return;
+    if (PARK) __syncthreads();  // every row read back before the rows are staged
     // node rj of element re: its x and y columns, in the half that holds the node
     const int re = lane / NSH, rj = lane - re * NSH;
     const bool task = lane < NE && re < nv;
