@@ -146,7 +146,7 @@ def kernel_name(fmt, shape, pairs=True, fast=False):
     meshes do; fast: the certified-elastic stress mode)."""
     import intpointsfem_amd as ipf
     tf = lambda b: "true" if b else "false"
-    return f"void k_residual_fmt<{shape}, {ipf.B_FORMATS.index(fmt)}, false, {tf(pairs)}, {tf(fast)}>"
+    return f"void k_residual_fmt<{shape}, {ipf.B_FORMATS.index(fmt)}, false, {tf(pairs)}, {tf(fast)}, false>"
 
 
 def launch_roofline(ctx, u, r, nrep, blocks, npts, neq, fmt, step_ms=None):
@@ -685,11 +685,6 @@ def main():
     nrep = max(3, min(args.steps, 20))
     blocks = sm.export_blocks()
     roof = launch_roofline(ctx, u, r, nrep, blocks, npts, neq, fmt0, step_ms=ms_per_step)
-    # one untimed ipf_residual_tangent: its k_copy (f_lin into r, neq doubles
-    # read and written) is the known-size dispatch that checks the PMC byte
-    # counters of a profiled run (the residual itself needs no copy)
-    ctx.residual_tangent(u, torch.empty_like(r))
-    ctx.synchronize()
     kname = kernel_name(fmt0, shape)
     traffic, valu_busy = profile_figures(args.mesh, kname)
     roofline = roofline_entry(roof, f"{kname} (one launch per element color)", traffic, valu_busy, npts)

@@ -475,14 +475,15 @@ void release_data(ipf_ctx* ctx) {
 // launches' own times add up; above, the element forces no longer stay in the
 // Infinity Cache and their write and read cost what the colored launches'
 // repeated r costs.  us per residual, colored -> element / node, one context
-// alone: Q2 14 k points 23.2 -> 9.7, 90 k 25.3 -> 12.3, 360 k 34.8 -> 27.3,
-// 810 k 58.6 -> 45.6, 1.44 M 82.7 -> 73.8, 5.8 M 253 -> 264.  Where several
+// alone: Q2 14 k points 20.3 -> 8.3, 90 k 22.4 -> 11.0, 360 k 31.2 -> 24.3,
+// 810 k 49.5 -> 44.2, 1.44 M 69.6 -> 68.4, 5.8 M 210 -> 230.  Where several
 // contexts keep the chip busy (three on three streams) the gain ends earlier:
-// Q2 90 k 12.6 -> 6.6, 360 k 18.4 -> 17.1, 810 k 34.3 -> 37.2, Q1 360 k 16.2 ->
-// 15.6, 640 k 23.4 -> 25.2, Q3 314 k 22.6 -> 18.4, 640 k 32.9 -> 35.0; products
-// the same.  A CG iteration (nine launches -> three) waits for itself either
-// way: Q2 14 k 23.8 -> 12.9, 90 k 29.1 -> 16.8, 1.44 M 100.6 -> 85.1, 2.7 M
-// 152 -> 144, 5.8 M 280 -> 315.
+// Q2 90 k 12.0 -> 7.8, 360 k 14.6 -> 13.9, 810 k 26.7 -> 31.5, Q1 360 k 15.1 ->
+// 12.6, 640 k 18.8 -> 21.0, Q3 314 k 18.4 -> 15.4, 640 k 27.1 -> 30.0; products
+// the same, with the tangent Q2 90 k 23.0 -> 14.2, 360 k 39.8 -> 38.6, 1.44 M
+// 146 -> 152 (and its product).  A CG iteration waits for itself either way:
+// Q2 14 k 22.3 -> 12.0, 90 k 27.7 -> 15.3, 360 k 46.5 -> 31.2, 1.44 M 98.8 ->
+// 83.1, 5.8 M 282 -> 317.
 constexpr int64_t kSplitPoints = 400000, kSplitPointsCg = 2000000;
 
 // The B formats of the element launches: geometric or compact FP64.

@@ -46,9 +46,8 @@ void launch_predict(const short* wbf, const float* par, const float* feat, int64
 }  // namespace mlp
 
 // Features (trial principal stresses over c, ln c, phi, psi, 1e3 alpha), exact
-// branch and 1e3 d_alpha of one point.  Only the eigenvalues of the trial
-// stress are wanted (spectral_ps's equal spectral's); the material's own
-// features come from the host.
+// branch and 1e3 d_alpha of one point.  Of the trial stress only the
+// eigenvalues are wanted; the material's own features come from the host.
 __device__ __forceinline__ void point_features(const double* e3, const double* ep, double alpha, const MatConst& m,
                                                float* __restrict__ f, int& label, float& target) {
     double s[6];

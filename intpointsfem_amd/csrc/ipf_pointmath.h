@@ -112,10 +112,11 @@ IPF_HD void eigvec_double(const double* s, double lam, V3& vec1, V3& vec2) {
 
 // ---------------------------------------------------------------- plane strain
 //
-// spectral_ps: spectral() for a tensor whose XZ and YZ components are +0 (the
-// trial stresses and elastic strains of plane strain: mu * 0.0, 0.0).  The
-// results equal spectral()'s bit for bit up to the sign of exact zeros; only
-// work on the zero components is left out:
+// spectral_ps: the reference's decomposition (FunctionsSpectralDecomp.h) of a
+// tensor whose XZ and YZ components are +0 (the trial stresses and elastic
+// strains of plane strain: mu * 0.0, 0.0).  The results are the reference's bit
+// for bit up to the sign of exact zeros; only work on the zero components is
+// left out:
 //   * normalize: +0 / maxel is a zero with the sign of maxel;
 //   * Gershgorin rows: |sxy + (+-0)| = |sxy|;
 //   * cubic and derivative: sxz^2 = syz^2 = +0 and 2 sxy sxz syz = +-0.
@@ -128,7 +129,8 @@ IPF_HD void eigvec_double(const double* s, double lam, V3& vec1, V3& vec2) {
 //     the xy minor the vector is (zero, zero, 1) with norm exactly 1, and in
 //     the other two branches its z component is a zero that the division by
 //     the (finite, >= 1) norm leaves unchanged.
-// Non-finite or degenerate cases (a zero minor, NaN) take the general code.
+// A simple eigenvector whose largest minor is zero, subnormal or not finite
+// takes the general eigvec_simple.
 
 // Quotients by one divisor and square roots, correctly rounded like the
 // operators (and so the same bits), without the operators' scaling of extreme
