@@ -106,10 +106,16 @@ k_assemble_K(GroupDev g, const double* __restrict__ dep, int64_t npad, const int
 // Bound by the products (34 instructions per pair and point, 45 of 64 lanes at
 // Q2, 136 of 192 at Q3) and the round trips position -> entry.  Residual,
 // tangent and assembly, before (with the clear of Kg) -> now: 201x150 Q2
-// 124 -> 76 us; 300x300 (from the stored dense B throughout) Q1 186 -> 84,
+// 124 -> 66 us; 300x300 (from the stored dense B throughout) Q1 186 -> 84,
 // Q2 586 -> 240, Q3 2,280 -> 728 us.
+// Registers for seven wavefronts per SIMD where one element fills a wavefront:
+// a color of a mesh of some ten thousand elements is then in flight at once
+// (Q2 84 VGPRs, five wavefronts -> 44, eight: 201x150 Q2 71 -> 66 us; no
+// spills).  Several elements share a wavefront's LDS rows at Q1, T1 and T2,
+// which that bound would spill; Q3's LDS allows four anyway.
+constexpr int pair_waves(int ce) { return ce * (ce + 2) / 8 > kWave / 2 ? 7 : 1; }
 template <int SHAPE, bool GEOM>
-__global__ void __launch_bounds__(kWave)
+__global__ void __launch_bounds__(kWave, pair_waves(shape_ce(SHAPE)))
 k_assemble_pairs(GroupDev g, const double* __restrict__ geo, const double* __restrict__ dep, int64_t npad,
                  const int* __restrict__ lidx, double* __restrict__ kg) {
     constexpr int NIP = shape_nip(SHAPE), CE = shape_ce(SHAPE), ET = shape_et(SHAPE), TP = shape_tp(SHAPE);
