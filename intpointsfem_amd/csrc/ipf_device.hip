@@ -245,8 +245,9 @@ struct ipf_ctx {
     int* dNodeR = nullptr;
     // element / node launches (ipf_split.h): the launch of each shape, the
     // nodes' element entries, the element forces.  dEf serves the calls of one
-    // stream at a time (split_stream); the CG's is its own (dEfS, with the
-    // solver buffers)
+    // stream at a time (split_stream); the CG and the step graph of ipf_newton,
+    // which wait for their work before they return, have their own (dEfS, with
+    // the CG's buffers)
     bool split_ok = false;
     int map_stride = 0;
     SplitDev split[SHAPE_COUNT];
@@ -2306,16 +2307,17 @@ int ipf_set_dirichlet_mask(ipf_ctx* ctx, const signed char* mask_host) {
 namespace {
 
 // The launches of ipf_residual_tangent on stream s: r = f_lin - B^T (w sigma)
-// and w Dep, fused per element launch (split: dEf is free to use) or color.
+// and w Dep, fused per element launch (ef: element forces that no other stream's
+// work uses -- dEf after split_stream, or the solver's dEfS) or, ef null, color.
 // Against strain, stress and force launches over the dense blocks (kept where
 // only those are stored), neither the dense B (432 bytes per point, twice) nor
 // the strains and stresses are read or written: with one product K v,
 // 1.44 M Q2 points 394 -> 167 us.
-void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStream_t s, bool split) {
+void residual_tangent_launches(ipf_ctx* ctx, const double* u, double* r, hipStream_t s, double* ef) {
     const int fmt = dep_format(ctx);
-    if (split && fmt != FMT_D64 && !ctx->update_mem) {
-        elem_launches(ctx, EL_DEP, fmt, elem_args(ctx, u, ctx->dEf), s);
-        node_launch(ctx, ctx->dEf, ctx->dFlin, r, s);
+    if (ef && fmt != FMT_D64 && !ctx->update_mem) {
+        elem_launches(ctx, EL_DEP, fmt, elem_args(ctx, u, ef), s);
+        node_launch(ctx, ef, ctx->dFlin, r, s);
         return;
     }
     if (fmt != FMT_D64) {
@@ -2388,10 +2390,13 @@ int cg_blocks(ipf_ctx* ctx, double* x, double rtol, int maxit, double bnorm, int
 // ipf_residual_tangent into r = dNr (and the FP32 copy of w Dep for the
 // FP32 geometric tangent), ||r||^2 over the free DoFs (scalar 6), the CG
 // start for K dNd = dNr with ||r||^2 in scalar 7, its first kCgBlock
-// iterations and ||r_cg||^2 (block partials).  The same kernels in the same order
-// as the eager iteration, so the iterates are the same bits.  nullptr when
+// iterations and ||r_cg||^2 (block partials).  The element forces of the residual
+// are the CG's own (dEfS), which its products use after it: work that other calls
+// have pending on another stream never shares a buffer with the replays.  The
+// results are the eager iteration's bits; between kSplitPoints and kSplitPointsCg
+// that one takes the residual's launches per color instead.  nullptr when
 // capture fails (the caller then runs the iteration eagerly).  Needs the
-// solver buffers (and dDep32 for FMT_G32) allocated.
+// solver and CG buffers (and dDep32 for FMT_G32) allocated.
 hipGraphExec_t newton_step_graph(ipf_ctx* ctx, const double* u) {
     if (!ctx->cap_stream && hipStreamCreate(&ctx->cap_stream) != hipSuccess) {
         ctx->cap_stream = nullptr;
@@ -2402,7 +2407,7 @@ hipGraphExec_t newton_step_graph(ipf_ctx* ctx, const double* u) {
         (void)hipGetLastError();
         return nullptr;
     }
-    residual_tangent_launches(ctx, u, ctx->dNr, s, cg_split(ctx));
+    residual_tangent_launches(ctx, u, ctx->dNr, s, cg_split(ctx) ? ctx->dEfS : nullptr);
     if (ctx->tfmt == FMT_G32) launch_to_f32(9 * ctx->npad, ctx->dDep, ctx->dDep32, s);
     masked_norm_launch(ctx, ctx->dNr, s);
     cg_start(ctx, ctx->dNr, ctx->dNd, 7, s);
@@ -2429,8 +2434,8 @@ int ipf_residual_tangent(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     if (!u_dev || !r_dev) return fail(ctx, IPF_EINVAL, "ipf_residual_tangent: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if ((rc = ensure_solver_buffers(ctx))) return rc;
-    residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream,
-                              dep_format(ctx) != FMT_D64 && ctx->npad <= kSplitPoints && split_stream(ctx));
+    const bool split = dep_format(ctx) != FMT_D64 && ctx->npad <= kSplitPoints && split_stream(ctx);
+    residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream, split ? ctx->dEf : nullptr);
     ctx->have_tangent = true;
     ctx->dep32_ok = false;
     if ((rc = ensure_dep32(ctx))) return rc;
