@@ -49,7 +49,7 @@ IPF_HD QuadMap quad_map(const double* X, double xi, double eta) {
     }
     QuadMap m;
     m.det = xx * ye - xe * yx;
-    const double inv = quot(1.0, recip(m.det));  // 1 / det
+    const double inv = quot(1.0, recip(m.det));  // 1 / det (not finite below 2^-1024, 0 included)
     m.a = ye * inv;
     m.b = -(yx * inv);
     m.c = -(xe * inv);

@@ -129,18 +129,22 @@ IPF_HD void eigvec_double(const double* s, double lam, V3& vec1, V3& vec2) {
 //     the xy minor the vector is (zero, zero, 1) with norm exactly 1, and in
 //     the other two branches its z component is a zero that the division by
 //     the (finite, >= 1) norm leaves unchanged.
-// A simple eigenvector whose largest minor is zero, subnormal or not finite
-// takes the general eigvec_simple.
+// A tensor with an entry outside [2^-480, 2^480] (a zero one included) is
+// normalised by the operators, and a simple eigenvector whose largest minor is
+// zero, subnormal or not finite takes the general eigvec_simple.
 
 // Quotients by one divisor and square roots, correctly rounded like the
 // operators (and so the same bits), without the operators' scaling of extreme
-// operands: a reciprocal with error e^3 from the hardware's (e <= 5e-8), the
-// quotient corrected by its exact remainder.  7 instructions instead of 11 and
-// the waits between them, 3 for every further quotient by the same divisor; 10
-// instead of 18 for a root.  For divisors, quotients and radicands between
-// 2^-1000 and 2^1000 (zero numerators included); stresses between 1e-150 and
-// 1e150 stay inside (their minors, products of two, are within 1e-300 and
-// 1e300 or exactly 0, which the callers keep out).
+// operands: a reciprocal with error e^3 from the hardware's (e <= 5e-8; the
+// series 1 + e + e^2 of 1 / (1 - e)), the quotient corrected by its exact
+// remainder (P. W. Markstein, IBM J. Res. Dev. 34, 1990); the root by
+// Goldschmidt's coupled iteration and two such corrections.  7 instructions
+// instead of 11 and the waits between them, 3 for every further quotient by the
+// same divisor; 10 instead of 18 for a root.  They hold where neither the
+// reciprocal nor the remainder overflows or loses bits below the normal range:
+// 1 / d for every normal d, n / d for n and d in [2^-480, 2^480], finite
+// radicands from 1.  (Below 2^-1024 the hardware's reciprocal is infinite and a
+// quotient NaN.)
 struct Recip {
     double d, r;
 };
@@ -214,7 +218,11 @@ IPF_HD void eigenvalues_newton_ps(double up, double lo, const double* s, double 
 
 // eigvec_simple with sxz = syz = +-0: the xy minor's vector is (0, 0, 1), and
 // in the other two branches the z component is a zero.  A vanishing or
-// non-finite largest minor takes the general code.
+// non-finite largest minor takes the general code.  v^2 stays finite: where s_xy
+// exceeds the rounding of s_xx and s_yy, lam is off them by its order or by an ulp
+// of the trace, so |v| = |s_xy / (s_xx - lam)| is at most about 2^53; below it
+// s_xx - lam is 0 or an ulp.  |v| under 2^-27 leaves a norm of exactly 1, whose
+// quotient is v itself.
 IPF_HD V3 eigvec_simple_ps(const double* s, double lam) {
     const double ax = s[XX] - lam, ay = s[YY] - lam, az = s[ZZ] - lam;
     const double d0 = ax * ay - s[XY] * s[XY];
@@ -267,11 +275,22 @@ IPF_HD void spectral_ps(double* s, double* ev, double* vec) {
     if (fabs(s[YY]) > fabs(maxel)) maxel = s[YY];
     if (fabs(s[ZZ]) > fabs(maxel)) maxel = s[ZZ];
     if (maxel != 0) {
+        const double least = fmin(fmin(fabs(s[XX]), fabs(s[XY])), fmin(fabs(s[YY]), fabs(s[ZZ])));
+        // Four quotients by recip, replaced where an entry is out of its range: a
+        // test per point (800x800: Q2 193.3 -> 194.8 us, Q3 443.9 -> 445.7; as an
+        // if / else before the quotients 196.5 and 451.3 against 195.0 and 448.3)
         const Recip m = recip(maxel);
-        s[XX] = quot(s[XX], m);
-        s[XY] = quot(s[XY], m);
-        s[YY] = quot(s[YY], m);
-        s[ZZ] = quot(s[ZZ], m);
+        double q0 = quot(s[XX], m), q1 = quot(s[XY], m), q2 = quot(s[YY], m), q3 = quot(s[ZZ], m);
+        if (!(least >= 0x1p-480 && fabs(maxel) <= 0x1p480)) {
+            q0 = s[XX] / maxel;
+            q1 = s[XY] / maxel;
+            q2 = s[YY] / maxel;
+            q3 = s[ZZ] / maxel;
+        }
+        s[XX] = q0;
+        s[XY] = q1;
+        s[YY] = q2;
+        s[ZZ] = q3;
         const double z = maxel > 0 ? 0.0 : (maxel < 0 ? -0.0 : s[XZ] / maxel);
         s[XZ] = z;
         s[YZ] = z;
