@@ -61,7 +61,7 @@ __device__ __forceinline__ void point_features(const double* e3, const double* e
     spectral_ps(s, ev, vec);
     int mt, br;
     project<false>(ev, sp, mt, br, hard, m, nullptr);
-    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));  // any float address
     f4* out = reinterpret_cast<f4*>(f);
     out[0] = f4{(float)(ev[0] / m.feat_c), (float)(ev[1] / m.feat_c), (float)(ev[2] / m.feat_c), m.feat_lnc};
     out[1] = f4{m.feat_phi, m.feat_psi, (float)(alpha * 1e3), 0.f};

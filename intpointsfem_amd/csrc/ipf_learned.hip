@@ -33,6 +33,7 @@ using namespace mlp;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a caller's features: any float address
 
 // round to nearest even (NaN kept quiet)
 __device__ __forceinline__ short f2bf(float x) {
@@ -126,8 +127,8 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
            double* __restrict__ loss_slots) {
     constexpr int NT = H / 16;
     __shared__ WeightsLDS w;
-    __shared__ float G[NPAR];
-    __shared__ short turn[4][16][OUTP];
+    __shared__ alignas(16) float G[NPAR];  // read back 16 bytes at a time
+    __shared__ alignas(8) short turn[4][16][OUTP];
     __shared__ double wave_loss[4];
     load_weights(w, wbf, par);
     __syncthreads();
@@ -168,7 +169,7 @@ k_mlp_grad(const short* __restrict__ wbf, const float* __restrict__ par, const f
         const int64_t s0 = tile * 16, q = s0 + r;
         // inputs: features 4g.. of sample r, and feature r of samples 4g..
         f32x4 xf = zero, xs = zero;
-        if (g < 2 && q < n) xf = *reinterpret_cast<const f32x4*>(feat + q * FEAT_STRIDE + 4 * g);
+        if (g < 2 && q < n) xf = *reinterpret_cast<const f32x4_any*>(feat + q * FEAT_STRIDE + 4 * g);
         if (g == 1) xf[3] = 0.f;  // IN = 7 features
 #pragma unroll
         for (int i = 0; i < 4; i++)
@@ -407,7 +408,7 @@ __device__ __forceinline__ f32x4 mfma_k32(bf16x4 a0, bf16x4 a1, bf16x4 b0, bf16x
 
 __device__ __forceinline__ f32x4 load_feat(const float* __restrict__ feat, int64_t q, int64_t n, int g) {
     f32x4 f = {0.f, 0.f, 0.f, 0.f};
-    if (g < 2 && q < n) f = *reinterpret_cast<const f32x4*>(feat + q * FEAT_STRIDE + 4 * g);
+    if (g < 2 && q < n) f = *reinterpret_cast<const f32x4_any*>(feat + q * FEAT_STRIDE + 4 * g);
     return f;
 }
 
