@@ -58,7 +58,10 @@ const char *ipf_last_error(const ipf_ctx *ctx);
 const char *ipf_global_last_error(void);
 
 /* Use a caller-owned stream (hipStream_t passed as void*); NULL restores the
- * context's own stream. */
+ * context's own stream.  Neither waits nor orders the two streams.  Call
+ * ipf_synchronize before leaving a stream, so that what the context lent to it
+ * (see ipf_residual) is free for the next; destroy a stream only after the
+ * work issued on it has ended. */
 int ipf_set_stream(ipf_ctx *ctx, void *hip_stream);
 void *ipf_get_stream(const ipf_ctx *ctx);
 int ipf_synchronize(ipf_ctx *ctx);
@@ -151,6 +154,12 @@ int ipf_set_update_mem(ipf_ctx *ctx, int update_mem);
  * device bytes held. */
 int ipf_info(const ipf_ctx *ctx, int64_t out[8]);
 
+/* How many calls of ipf_residual (colored assembly), ipf_residual_tangent,
+ * ipf_tangent_apply and ipf_multiply_transpose on this context took the
+ * element and node launches (out[0]) and the launches per color (out[1]); see
+ * ipf_residual for the rule. */
+int ipf_launch_routes(const ipf_ctx *ctx, int64_t out[2]);
+
 /* ---- the hot path ---- */
 
 /* r = f_lin - sum_e B_e^T (w * sigma(B_e u_e)), device pointers [neq].
@@ -158,11 +167,16 @@ int ipf_info(const ipf_ctx *ctx, int64_t out[8]);
  * (TPZElastoPlasticIntPointsStructMatrix.cpp:137-154) ->
  * TPZNumericalIntegrator::ResidualIntegration (TPZNumericalIntegrator.cpp:107-128).
  * One fused kernel per element color: gather, B.u, return map, B^T (w sigma)
- * and the color's atomic-free accumulation into r -- or, up to 400,000
- * points of geometric or compact FP64 B with aligned (x, y) DoF pairs in at most 8 colors, one
- * element launch per shape and one node launch that sums in color order (the
- * same bits; calls that overlap on several streams, and calls under capture,
- * keep the launch per color).  r is overwritten entirely (its previous contents are never read); u and r must not
+ * and the color's atomic-free accumulation into r -- or, up to 400,000 points
+ * of geometric or compact FP64 B with aligned (x, y) DoF pairs in at most 8
+ * colors, one element launch per shape and one node launch that sums in color
+ * order (the same bits).  Those two share a buffer of element forces, lent to
+ * the first stream that uses it until ipf_synchronize has waited for that
+ * stream: calls on another stream meanwhile, calls on hipStreamPerThread and
+ * calls under capture keep the launch per color.  (400,000: where several
+ * contexts keep the GPU busy at once the gain ends about there; a context
+ * alone would still gain some percent up to about a million points.)  r is
+ * overwritten entirely (its previous contents are never read); u and r must not
  * overlap.  Asynchronous on the context's stream. */
 int ipf_residual(ipf_ctx *ctx, const double *u_dev, double *r_dev);
 int ipf_residual_host(ipf_ctx *ctx, const double *u_host, double *r_host);

@@ -97,6 +97,7 @@ def lib():
         "ipf_set_rhs_linear": (_int, [_vp, _dp]),
         "ipf_set_update_mem": (_int, [_vp, _int]),
         "ipf_info": (_int, [_vp, _lp]),
+        "ipf_launch_routes": (_int, [_vp, _lp]),
         "ipf_residual": (_int, [_vp, _vp, _vp]),
         "ipf_residual_host": (_int, [_vp, _dp, _dp]),
         "ipf_residual_timed": (_int, [_vp, _vp, _vp, _dp, _lp, _int]),
@@ -485,6 +486,12 @@ class DeviceContext:
         self._c(lib().ipf_info(self._h, _p(out, _lp)), "ipf_info")
         keys = ("nblocks", "npts", "rows", "cols", "neq", "ncolor", "nstorage", "device_bytes")
         return dict(zip(keys, (int(v) for v in out)))
+
+    def launch_routes(self):
+        """(calls by element and node launches, calls by launches per color) so far."""
+        out = (_i64 * 2)()
+        self._c(lib().ipf_launch_routes(self._h, out), "ipf_launch_routes")
+        return out[0], out[1]
 
     # ---- compute on device pointers (torch tensors or raw ints)
     def residual(self, u, r):

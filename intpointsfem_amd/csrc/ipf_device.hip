@@ -255,6 +255,8 @@ struct ipf_ctx {
     int* dMap = nullptr;
     double* dEfS = nullptr;
     int64_t nent = 0;           // node entries of all element slots
+    // calls by route: the element / node launches, the launches per color
+    int64_t routes[2] = {0, 0};
     bool ef_bound = false;
     hipStream_t ef_stream = nullptr;
     double* dU = nullptr;       // staging for host-pointer calls: u, then r (dR)
@@ -874,6 +876,22 @@ void stress_launches(ipf_ctx* ctx, const double* strain, double* wsigma, double*
                      ctx->dOrig, st, ctx->stream);
 }
 
+// r = f_lin - B^T(w sigma) by the colored assembly's launches, in the residual's
+// format: element / node launches or, in color order, one per group.
+void residual_launches(ipf_ctx* ctx, const double* u, double* r) {
+    const bool split = !ctx->update_mem && split_format(ctx, ctx->rfmt) && ctx->npad <= kSplitPoints && split_stream(ctx);
+    ctx->routes[split ? 0 : 1]++;
+    if (split) {
+        elem_launches(ctx, ctx->residual_mode == IPF_RESIDUAL_CERTIFIED_ELASTIC ? EL_CERTIFIED : EL_RESIDUAL, ctx->rfmt,
+                      elem_args(ctx, u, ctx->dEf), ctx->stream);
+        node_launch(ctx, ctx->dEf, ctx->dFlin, r, ctx->stream);
+        return;
+    }
+    const double* flin = residual_start(ctx, r);
+    const PointState st = point_state(ctx);
+    for (const auto& g : ctx->groups) launch_group_residual(ctx, g, u, r, flin, st);
+}
+
 // y = K v on stream s: the tangent launches of every group in the selected
 // B format.  When every DoF has a first write (fold_flin), the flagged entries
 // start from 0 and y needs no clear; else y is cleared first.
@@ -887,6 +905,15 @@ void tangent_product(ipf_ctx* ctx, const double* v, double* y, hipStream_t s) {
         launch_tangent_fmt(ctx->tfmt, g.shape, d, group_fmt_B(ctx, g, ctx->tfmt), v, y, ctx->dDep, ctx->dDep32,
                            ctx->npad, zf, s);
     }
+}
+
+// y = K v on the context's stream: element / node launches, else tangent_product.
+void product_launches(ipf_ctx* ctx, const double* v, double* y) {
+    const bool split = split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPoints && split_stream(ctx);
+    ctx->routes[split ? 0 : 1]++;
+    if (!split) return tangent_product(ctx, v, y, ctx->stream);
+    elem_launches(ctx, EL_TANGENT, ctx->tfmt, elem_args(ctx, v, ctx->dEf), ctx->stream);
+    node_launch(ctx, ctx->dEf, nullptr, y, ctx->stream);
 }
 
 // The FP32 copy of w Dep the FMT_G32 tangent product reads, made after each
@@ -1146,6 +1173,13 @@ int ipf_info(const ipf_ctx* ctx, int64_t out[8]) {
     out[5] = ctx->ncolor;
     out[6] = ctx->nstorage;
     out[7] = ctx->bytes;
+    return IPF_OK;
+}
+
+int ipf_launch_routes(const ipf_ctx* ctx, int64_t out[2]) {
+    if (!ctx || !out) return fail(nullptr, IPF_EINVAL, "ipf_launch_routes: null argument");
+    out[0] = ctx->routes[0];
+    out[1] = ctx->routes[1];
     return IPF_OK;
 }
 
@@ -1958,17 +1992,7 @@ int ipf_residual(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     if (!u_dev || !r_dev) return fail(ctx, IPF_EINVAL, "ipf_residual: NULL pointer");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if (ctx->assembly == IPF_ASSEMBLY_PATCH && !ctx->update_mem) return patch_residual(ctx, u_dev, r_dev);
-    if (!ctx->update_mem && split_format(ctx, ctx->rfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
-        elem_launches(ctx, ctx->residual_mode == IPF_RESIDUAL_CERTIFIED_ELASTIC ? EL_CERTIFIED : EL_RESIDUAL, ctx->rfmt,
-                      elem_args(ctx, u_dev, ctx->dEf), ctx->stream);
-        node_launch(ctx, ctx->dEf, ctx->dFlin, r_dev, ctx->stream);
-        return launch_status(ctx, "residual");
-    }
-    // r = f_lin, then each color adds -B^T(w sigma)
-    const double* flin = residual_start(ctx, r_dev);
-    const PointState st = point_state(ctx);
-    for (const auto& g : ctx->groups)
-        launch_group_residual(ctx, g, u_dev, r_dev, flin, st);
+    residual_launches(ctx, u_dev, r_dev);
     return launch_status(ctx, "residual");
 }
 
@@ -2162,8 +2186,10 @@ int ipf_multiply_transpose(ipf_ctx* ctx, const double* wsigma_dev, double* res_d
         a.point = const_cast<double*>(wsigma_dev);  // read only
         elem_launches(ctx, EL_FORCE, dep_format(ctx), a, ctx->stream);
         node_launch(ctx, ctx->dEf, nullptr, res_dev, ctx->stream);
+        ctx->routes[0]++;
         return launch_status(ctx, "multiply_transpose");
     }
+    ctx->routes[1]++;
     launch_fill(ctx->neq, res_dev, 0.0, ctx->stream);
     for (const auto& g : ctx->groups)
         launch_transpose(g.shape, group_dev(ctx, g), wsigma_dev, res_dev, ctx->dOrig, ctx->stream);
@@ -2435,6 +2461,7 @@ int ipf_residual_tangent(ipf_ctx* ctx, const double* u_dev, double* r_dev) {
     IPF_HIP(ctx, hipSetDevice(ctx->device));
     if ((rc = ensure_solver_buffers(ctx))) return rc;
     const bool split = dep_format(ctx) != FMT_D64 && ctx->npad <= kSplitPoints && split_stream(ctx);
+    ctx->routes[split && !ctx->update_mem ? 0 : 1]++;
     residual_tangent_launches(ctx, u_dev, r_dev, ctx->stream, split ? ctx->dEf : nullptr);
     ctx->have_tangent = true;
     ctx->dep32_ok = false;
@@ -2629,12 +2656,7 @@ int ipf_tangent_apply(ipf_ctx* ctx, const double* v_dev, double* y_dev) {
     if (!v_dev || !y_dev) return fail(ctx, IPF_EINVAL, "ipf_tangent_apply: NULL pointer");
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    if (split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPoints && split_stream(ctx)) {
-        elem_launches(ctx, EL_TANGENT, ctx->tfmt, elem_args(ctx, v_dev, ctx->dEf), ctx->stream);
-        node_launch(ctx, ctx->dEf, nullptr, y_dev, ctx->stream);
-    } else {
-        tangent_product(ctx, v_dev, y_dev, ctx->stream);
-    }
+    product_launches(ctx, v_dev, y_dev);
     return launch_status(ctx, "tangent_apply");
 }
 
