@@ -155,9 +155,9 @@ int ipf_set_update_mem(ipf_ctx *ctx, int update_mem);
 int ipf_info(const ipf_ctx *ctx, int64_t out[8]);
 
 /* How many calls of ipf_residual (colored assembly), ipf_residual_tangent,
- * ipf_tangent_apply and ipf_multiply_transpose on this context took the
- * element and node launches (out[0]) and the launches per color (out[1]); see
- * ipf_residual for the rule. */
+ * ipf_tangent_apply and ipf_multiply_transpose on this context, and timed
+ * repetitions of ipf_autotune, took the element and node launches (out[0])
+ * and the launches per color (out[1]); see ipf_residual for the rule. */
 int ipf_launch_routes(const ipf_ctx *ctx, int64_t out[2]);
 
 /* ---- the hot path ---- */
@@ -342,7 +342,8 @@ int ipf_set_b_format(ipf_ctx *ctx, int residual_format, int tangent_format);
  * state untouched) in every exact FP64 form the data allows (dense, compact,
  * geometric) and, after ipf_residual_tangent, the tangent product likewise
  * (with allow_fp32, also the FP32 forms: the CG matvecs then steer an FP64
- * Newton, see above), and selects the fastest of each.  The FP64 forms give
+ * Newton, see above), by the launches that the calls take -- the product's, up
+ * to 2,000,000 points, those of the CG -- and selects the fastest of each.  The FP64 forms give
  * bit-identical results, so the choice changes only the time.  times_ms
  * (optional) [2 * 6]: average ms per residual by format, then per tangent
  * product by format, -1 where not timed (format codes as above).  Frees

@@ -907,9 +907,10 @@ void tangent_product(ipf_ctx* ctx, const double* v, double* y, hipStream_t s) {
     }
 }
 
-// y = K v on the context's stream: element / node launches, else tangent_product.
-void product_launches(ipf_ctx* ctx, const double* v, double* y) {
-    const bool split = split_format(ctx, ctx->tfmt) && ctx->npad <= kSplitPoints && split_stream(ctx);
+// y = K v on the context's stream: element / node launches up to max_points
+// points, else tangent_product.
+void product_launches(ipf_ctx* ctx, const double* v, double* y, int64_t max_points) {
+    const bool split = split_format(ctx, ctx->tfmt) && ctx->npad <= max_points && split_stream(ctx);
     ctx->routes[split ? 0 : 1]++;
     if (!split) return tangent_product(ctx, v, y, ctx->stream);
     elem_launches(ctx, EL_TANGENT, ctx->tfmt, elem_args(ctx, v, ctx->dEf), ctx->stream);
@@ -2256,13 +2257,7 @@ int ipf_autotune(ipf_ctx* ctx, const double* u_dev, int reps, int allow_fp32, do
         double ms;
         if (!fp32) {
             ctx->rfmt = f;
-            rc = time_it(
-                [&] {
-                    const double* flin = residual_start(ctx, ctx->dR);
-                    for (const auto& g : ctx->groups)
-                        launch_group_residual(ctx, g, u_dev, ctx->dR, flin, point_state(ctx));
-                },
-                &ms);
+            rc = time_it([&] { residual_launches(ctx, u_dev, ctx->dR); }, &ms);
             if (rc) break;
             if (times_ms) times_ms[f] = ms;
             if (ms < tr) tr = ms, best_r = f;
@@ -2270,11 +2265,8 @@ int ipf_autotune(ipf_ctx* ctx, const double* u_dev, int reps, int allow_fp32, do
         if (ctx->have_tangent && (!fp32 || allow_fp32)) {
             ctx->tfmt = f;
             if ((rc = ensure_dep32(ctx))) break;
-            rc = time_it(
-                [&] {
-                    tangent_product(ctx, u_dev, ctx->dR, ctx->stream);
-                },
-                &ms);
+            // as a CG forms its products, the most of them
+            rc = time_it([&] { product_launches(ctx, u_dev, ctx->dR, kSplitPointsCg); }, &ms);
             if (rc) break;
             if (times_ms) times_ms[FMT_COUNT + f] = ms;
             if (ms < tt) tt = ms, best_t = f;
@@ -2656,7 +2648,7 @@ int ipf_tangent_apply(ipf_ctx* ctx, const double* v_dev, double* y_dev) {
     if (!v_dev || !y_dev) return fail(ctx, IPF_EINVAL, "ipf_tangent_apply: NULL pointer");
     if (!ctx->have_tangent) return fail(ctx, IPF_ESTATE, "no tangent: call ipf_residual_tangent first");
     IPF_HIP(ctx, hipSetDevice(ctx->device));
-    product_launches(ctx, v_dev, y_dev);
+    product_launches(ctx, v_dev, y_dev, kSplitPoints);
     return launch_status(ctx, "tangent_apply");
 }
 

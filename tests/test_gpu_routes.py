@@ -7,6 +7,7 @@ Bars: a call on the context's first stream takes the element / node launches,
 the same call on a second one (the first not waited for by ipf_synchronize) the
 launches per color, and both give the same bits; strains and stresses are the
 oracle's bit for bit; a CG solution's own residual ||b - K x|| <= 10 rtol ||b||.
+ipf_autotune times the launches that the calls take.
 """
 import os
 
@@ -158,3 +159,28 @@ def test_triangles_and_quadrilaterals(gpu, p, ncolor, source):
     ctx.synchronize()
     res = np.where(part.fixed, 0.0, b - y.cpu().numpy())
     assert np.linalg.norm(res) <= 10 * rtol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("mesh", [(12, 10, 2, 1.1), (7, 5, 3, 1.1)], ids=str)
+def test_autotune_times_the_launches_of_the_calls(gpu, mesh):
+    import torch
+    m = wb.make_mesh(mesh)
+    sm = ipf.StructMatrix(m, device=0)
+    ctx = sm.context()
+    u = torch.as_tensor(wb.lame_displacement(m.nodes(), wb.normal_stress(10)), dtype=torch.float64, device=gpu)
+    r = torch.zeros_like(u)
+    torch.cuda.synchronize()
+    ctx.residual_tangent(u, r)
+    reps = 10
+    before = ctx.launch_routes()
+    t = ctx.autotune(u, reps=reps, allow_fp32=True)
+    after = ctx.launch_routes()
+    # element / node launches: compact and geometric FP64 (and FP32 geometric
+    # for the product); the other forms have launches per color only
+    split = sum(f in ("compact-fp64", "geometry-fp64") for f in t["residual"])
+    split += sum(f in ("compact-fp64", "geometry-fp64", "geometry-fp32") for f in t["tangent"])
+    per_color = len(t["residual"]) + len(t["tangent"]) - split
+    assert split == 5 and per_color == 4
+    assert (after[0] - before[0], after[1] - before[1]) == (split * (reps + 2), per_color * (reps + 2))
+    # two launches against four: the choice stays with the forms that have them
+    assert t["selected"][0] in ("compact-fp64", "geometry-fp64")
