@@ -166,6 +166,10 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
         us[2 * lane + 1] = uy;
     }
     if (POINTS && slot && lane == el * C::NIP) oel[el] = o;
+    // returned strains and forces keep what the blocks' zeros make of an
+    // infinite or NaN value (a return map makes NaN of such a point anyway)
+    const bool odd_u =
+        OP == EL_STRAIN && __ballot(!(__builtin_isfinite(ux) && __builtin_isfinite(uy))) != 0;
     __syncthreads();
     if constexpr (OP == EL_FORCE) {
         load_points<3, C::NIP>(pts, oel, nv, a.point);
@@ -179,9 +183,18 @@ k_elem(SplitDev g, const double* __restrict__ u, ElemArgs a) {
         if constexpr (OP == EL_STRAIN) {
 #pragma unroll
             for (int k = 0; k < 3; k++) pts[3 * lane + k] = e3[k];
+            if (odd_u) {
+                for (int a = 0; a < NSH; a++) {
+                    pts[3 * lane] += 0.0 * us[el * C::CE + 2 * a + 1];
+                    pts[3 * lane + 2] += 0.0 * us[el * C::CE + 2 * a];
+                }
+            }
         } else if constexpr (OP == EL_FORCE) {
 #pragma unroll
             for (int k = 0; k < 3; k++) x[k] = pts[3 * lane + k];
+            const double xx = x[0];
+            x[0] += 0.0 * x[2];
+            x[2] += 0.0 * xx;
         } else if constexpr (FEAT) {
             point_features(e3, ep, alpha, g.mats[tm >> 8], a.feat + o * mlp::FEAT_STRIDE, a.label[o], a.target[o]);
         } else if constexpr (TAN) {
